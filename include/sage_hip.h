@@ -67,7 +67,9 @@ typedef enum sage_pv_accum { SAGE_PV_F32 = 0, SAGE_PV_F16 = 1 } sage_pv_accum;
  * behind) over the same 128 queries; every other tile, the defaults included,
  * runs four wave64s of 32 queries, each doing the whole block. Both
  * double-buffer K and V. KV-merged attention always runs the four-wave
- * layout. */
+ * layout. Grids of too few query tiles to fill the chip run, under every tile,
+ * a third layout that splits the keys over a workgroup's waves; its outputs
+ * differ from the others' by the order of fp32 sums alone. */
 typedef struct sage_tile {
     uint32_t warps;
     uint32_t m_tiles;
@@ -224,8 +226,8 @@ void* sage_stream(const sage_attention* s);                  /* mod.rs:636-638 *
 
 /* attn_resources (mod.rs:640-646): VGPRs per lane and scratch (spill) bytes
  * of the attention kernel, plus its static LDS bytes. The kernel is the one
- * the context's tile selects: the eight-wave layout for warps 8, else the
- * four-wave kernel. */
+ * the context's tile selects on grids that fill the chip: the eight-wave
+ * layout for warps 8, else the four-wave kernel. */
 sage_status sage_attn_resources(const sage_attention* s, int32_t* regs, int32_t* spill, int32_t* lds);
 
 /* The same for each attention kernel the context can launch (extension: the

@@ -47,6 +47,7 @@ UNITS = [
     ("sage_prologue.hip", "sage_prologue.hip.o", ["-ffp-contract=off"]),
     ("sage_attention.hip", "sage_attention.hip.o", SCHED),
     ("sage_attention.hip", "sage_attention_merged.hip.o", ["-DSAGE_ATTN_MERGED"]),
+    ("sage_attn_keys.hip", "sage_attn_keys.hip.o", []),
     ("sage_peak.hip", "sage_peak.hip.o", []),
     ("sage_noalloc.hip", "sage_noalloc.hip.o", []),
     ("sage_api.cpp", "sage_api.cpp.o", []),

@@ -47,97 +47,10 @@
 //   in LDS beside K and V. The log2 logit x = S * sc + bias is formed before
 //   the row max (fmaf(1.5 * 2^23 + S, sc, fmaf(-1.5 * 2^23, sc, bias))), and
 //   P = 2^(x + log2(448) - m); padding keys carry -inf and need no mask.
-#include "sage_device.hpp"
+#include "sage_attn_device.hpp"
 #include "sage_internal.hpp"
 
 namespace sage {
-
-constexpr int ATTN_BN = 64;  // keys per iteration (one K scale, one V block)
-constexpr int MAGIC_BITS = 0x4B400000;      // bits of 1.5 * 2^23
-constexpr float MAGIC = 12582912.0f;        // 1.5 * 2^23
-constexpr int NEG_INF_BITS = (int)0xFF800000;  // -inf: below every biased score as an int
-constexpr float LOG2_448 = 8.807354922057604f;  // P = 448 for the row max: E4M3's largest finite
-
-// A row statistic held in lane l and its partner lane l ^ 32 (the other half
-// of the wave), combined in every lane with one v_permlane32_swap of two copies
-// of x: the swap's first result holds the lower half's values in both halves,
-// its second the upper half's, so every lane combines the same pair in the
-// same order.
-__device__ __forceinline__ int max_halves(int x) {
-    const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
-    return max((int)r[0], (int)r[1]);
-}
-__device__ __forceinline__ float fmax_halves(float x) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(x), __float_as_int(x), false, false);
-    // v_med3_f32 with FLT_MAX: the maximum of two non-NaN values without the
-    // canonicalising v_max_f32 that fmaxf puts on each swapped register.
-    return __builtin_amdgcn_fmed3f(__int_as_float((int)r[0]), __int_as_float((int)r[1]), 3.4028234663852886e38f);
-}
-__device__ __forceinline__ float sum_halves(float x) {
-    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_int(x), __float_as_int(x), false, false);
-    return __int_as_float((int)r[0]) + __int_as_float((int)r[1]);
-}
-// Floor of the logit scale q_scale * k_scale in masked blocks: a masked score
-// is -inf and must stay -inf through the product (0 * -inf would be a NaN),
-// so the product is floored where scores are masked. Below 1e-30
-// the floor changes no result: every logit difference of the block is then
-// under 2^22 * 1e-30 < 1e-23, far below half an ulp of the exp2 argument
-// (about 8.8, ulp 2^-20), so every P and alpha come out bit-identical to the
-// unfloored product's. Only an exact zero scale (an all-zero 16-row Q group,
-// a K head constant over tokens) is changed: the row attends uniformly to its
-// visible keys, where the reference's masked keys turn into NaNs.
-constexpr float SCALE_FLOOR = 1.0e-30f;
-// max(m, x) for the running max: v_med3_f32(m, x, FLT_MAX) in one instruction
-// (fmaxf on the loop-carried m costs a canonicalising v_max_f32 m, m every
-// block). Neither operand is a NaN: m starts at -1e30 and x is a finite logit
-// or -inf.
-__device__ __forceinline__ float running_max(float m, float x) {
-    return __builtin_amdgcn_fmed3f(m, x, 3.4028234663852886e38f);
-}
-// Values the compiler may not re-derive or rematerialise: a uniform pointer
-// stays in SGPRs and is not reassociated with per-lane offsets; a VGPR value
-// stays where it is. (The constraints name AMDGPU register classes, so the
-// statements exist only in the device pass.)
-__device__ __forceinline__ const uint8_t* opaque_uniform(const uint8_t* p) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("" : "+s"(p));
-#endif
-    return p;
-}
-template <typename T>
-__device__ __forceinline__ void opaque_vgpr(T& x) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("" : "+v"(x));
-#endif
-}
-
-// The dispatcher deals workgroups to the 8 XCDs round-robin by linear id,
-// and each XCD has its own L2. Tile t (query tile fastest, then head, then
-// batch) goes to the workgroup that gives XCD x the contiguous range of
-// tiles [x * per, (x + 1) * per): the workgroups that share a head's K and V
-// then read them through one L2 instead of eight. The last total % 8 tiles
-// keep their place.
-__device__ __forceinline__ int xcd_tile(int lin, int total) {
-    const int per = total / NUM_XCD;
-    if (lin >= per * NUM_XCD) return lin;
-    return (lin % NUM_XCD) * per + lin / NUM_XCD;
-}
-
-// A causal query tile qt sweeps 2 qt + 2 key blocks. Dealt head by head,
-// the heavy tiles of an XCD's last head start late and finish alone; dealt
-// longest first across the XCD's heads, the short tiles fill the tail. That
-// order needs every XCD to hold whole heads (the plain mapping above does
-// then too, so the L2 sharing is unchanged).
-__device__ __forceinline__ bool causal_longest_first(int total, int ntq) {
-    return total % NUM_XCD == 0 && (total / NUM_XCD) % ntq == 0;
-}
-
-// This lane's index in the wave, rebuilt from v_mbcnt: values derived from the
-// lane are recomputed where a rare path or the epilogue needs them instead of
-// being kept live (or spilled) across the key loop.
-__device__ __forceinline__ int lane_now() {
-    return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
-}
 
 // Workgroups a CU: four at head dim 64 (<= 128 VGPRs), three at head dim 128
 // (<= 168); the merged head-dim-128 kernel needs the registers of two.
@@ -874,9 +787,44 @@ static hipError_t resources_of(int head_dim, int* regs, int* spill, int* lds) {
 // default order and are built in the second pass.
 #ifndef SAGE_ATTN_MERGED
 
+// How many shares the keys of a query group are split into (sage_attn_keys),
+// or 0 for the whole-key kernels, by the number of 128-query tiles: n / 256 a
+// CU. A tile is one wave a SIMD, and a lone wave takes 1.6 times the chip's
+// best time a block, so up to n = 256 the chip is short of waves however long
+// the keys; a split has more of them but reads K and V once per 32 or 64
+// queries instead of 128 and sweeps the keys' first shares twice (15 to 20%
+// slower at head dim 64 on a full chip, 30 to 35% at 128, where its LDS holds
+// two waves a SIMD). Measured (us, whole keys / four shares / two):
+//   D 64        96 tiles N 689: 11.8 / 8.0 / 9.1     176, N 1378: 19.9 / 16.7 / 19.0
+//               256, N 1000: 16.7 / 16.3 / 15.9      352, N 2756: 52.5 / 48.1 / 46.3
+//               384, N 2048: 40.7 / 38.6 / 36.4      480, N 5000: 92.1 / 104 / 95.2
+//   D 64 causal 256, N 1000: 16.3 / 11.5 / 12.9      352, N 2756: 36.2 / 27.6 / 28.6
+//               480, N 5000: 81.3 / 67.8 / 63.2      704, N 5512: 78.5 / 84.5 / 79.8
+//   D 128       128, N 8192: 118 / 76.9 / 84.7       176, N 1378: 27.6 / 27.5 / 27.8
+//               256, N 1000: 23.2 / 28.5 / 24.1
+//   D 128 causal 176, N 1378: 26.8 / 20.7 / 21.2     256, N 1000: 22.3 / 21.5 / 18.9
+//               352, N 2756: 49.3 / 47.7 / 43.9      384, N 689: 18.0 / 24.5 / 21.8
+//   merged      D 64 96 tiles, stride 2: 7.2 / 6.2 / 6.4, stride 4: 5.5 / 5.7 / 5.3;
+//               D 128 96, stride 2: 9.8 / 8.6 / 8.7, stride 4: 8.2 / 8.2 / 7.1;
+//               352 D 64: 21.9 / 23.4 / 21.9, D 128: 29.8 / 41.5 / 37.9
+// (A causal tile's keys end at its queries, so causal grids carry half the
+// work and longer tails. The tile of the context's Config does not matter
+// here: it picks a layout, never a result.)
+static int key_shares(int head_dim, const Geom& g) {
+    const long long n = (long long)g.q_tiles * g.heads * g.batch;
+    if (g.merge > 1) return n <= (head_dim == 64 ? 224 : 128) ? 2 : 0;
+    if (head_dim == 64) {
+        if (g.flags & F_CAUSAL) return n <= 320 ? 4 : n <= 560 ? 2 : 0;
+        return n <= 224 ? 4 : n <= 416 ? 2 : 0;
+    }
+    if (g.flags & F_CAUSAL) return n <= 208 ? 4 : n <= 320 ? 2 : 0;
+    return n <= 160 ? 4 : 0;
+}
+
 // Dense, causal (an extension) or merged (sg_attn_merge); the API refuses
 // causal masking over merged keys.
 hipError_t launch_attention(int head_dim, const AttendBufs& w, const Geom& g, hipStream_t s) {
+    if (const int shares = key_shares(head_dim, g)) return launch_attention_keys(head_dim, shares, w, g, s);
     if (g.merge > 1) return launch_attention_merged(head_dim, w, g, s);
     if (g.flags & F_WAVES8) {
         if (head_dim == 64)

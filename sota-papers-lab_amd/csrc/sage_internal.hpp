@@ -63,6 +63,9 @@ hipError_t launch_attention(int head_dim, const AttendBufs& w, const Geom& g, hi
 // The merged kernels' launch, from the second compilation of the attention
 // source (launch_attention calls it for merged plans).
 hipError_t launch_attention_merged(int head_dim, const AttendBufs& w, const Geom& g, hipStream_t s);
+// The keys-split kernels' launch, two or four shares of the keys a query
+// group (launch_attention calls it for grids of few query tiles).
+hipError_t launch_attention_keys(int head_dim, int shares, const AttendBufs& w, const Geom& g, hipStream_t s);
 
 // Kernel resources (VGPRs, scratch, LDS) of the attention kernel for
 // head_dim: dense, causal or KV-merged; waves8 = the eight-wave layout that

@@ -1,0 +1,74 @@
+"""The attention kernels on both sides of the line between split and whole keys.
+
+Grids of few query tiles run the kernel that splits a query group's keys over
+two or four waves; larger ones the whole-key kernels. Each case sits at a place
+where the split can go wrong: fewer key blocks than shares, a ragged last
+block, blocks past the 64 whose scales a wave holds at a time, causal groups
+whose last share is the diagonal alone, grouped heads, merged biases, and a
+running maximum that moves in the last share (token 0.9 N scaled up). The cases
+over the line keep the whole-key kernels' own masks and tails covered, the
+eight-wave layout among them. The gate is the fuzz test's: 2e-2 plus half an
+output step of the emulated reference arithmetic, and no further from f64.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from sage_gpu_helpers import run, sample_rows
+from test_gpu_fuzz import _check
+
+pytestmark = pytest.mark.gpu
+
+SPLIT = [
+    # batch, heads, tokens, head_dim, extra Problem arguments
+    (1, 1, 63, 64, {}),                                  # one ragged block, three empty shares
+    (1, 3, 129, 128, {}),                                # three blocks on four shares
+    (2, 5, 257, 64, dict(kv_heads=1, dtype=1)),
+    (1, 1, 4500, 64, {}),                                # 71 blocks: two chunks of K scales
+    (1, 1, 8200, 128, dict(dtype=1)),                    # 129 blocks, the last one of 8 keys
+    (1, 40, 1000, 64, {}),                               # two shares (320 tiles)
+    (1, 2, 4170, 128, dict(causal=True)),
+    (3, 4, 700, 64, dict(kv_heads=2, causal=True)),
+    (1, 8, 1000, 64, dict(causal=True)),                 # dealt longest first
+    (1, 48, 1100, 64, dict(causal=True, dtype=1)),       # two shares (432 tiles)
+    (1, 32, 1050, 128, dict(kv_heads=4, causal=True)),   # two shares (288 tiles)
+    (1, 3, 3 * 95, 64, dict(merge=2, layout=(3, 5, 9, 10, 1))),
+    (2, 2, 50 * 95, 128, dict(merge=4, layout=(50, 5, 9, 10, 0))),
+]
+WHOLE = [
+    (1, 54, 1000, 64, {}),
+    (1, 21, 1000, 128, dict(dtype=1)),
+    (1, 72, 1001, 64, dict(kv_heads=9, causal=True)),
+    (2, 20, 1050, 128, dict(causal=True)),
+    (1, 19, 16 * 95, 64, dict(merge=2, layout=(16, 5, 9, 10, 0))),
+    (1, 11, 16 * 95, 128, dict(merge=2, layout=(16, 5, 9, 10, 2))),
+]
+
+
+def _problem(oracle, b, h, n, d, kw, seed):
+    p = oracle.Problem(b, h, n, d, **kw)
+    q, k, v = oracle.generate(p, oracle.GenSpec(k_off_std=2.0, seed=seed))
+    # A late key that outgrows every row's maximum so far.
+    t = int(0.9 * n)
+    k[:, t] = oracle.encode16(2.0 * oracle.decode16(k[:, t], p.dtype), p.dtype)
+    return p, q, k, v
+
+
+@pytest.mark.parametrize("b,h,n,d,kw", SPLIT + WHOLE, ids=[f"b{c[0]}h{c[1]}n{c[2]}d{c[3]}" for c in SPLIT + WHOLE])
+def test_against_reference_arithmetic(oracle, torch_gpu, b, h, n, d, kw):
+    p, q, k, v = _problem(oracle, b, h, n, d, kw, 100 + n + d)
+    _, o = run(torch_gpu, p, q, k, v, want_ws=False)
+    rows = sample_rows(n, max(8, 4096 // (b * h)), seed=n)
+    _check(oracle, p, oracle.prologue(p, q, k, v), o, rows, q, k, v, p.dtype, f"b{b} h{h} n{n} d{d} {kw}")
+
+
+@pytest.mark.parametrize("b,h,n,d,kw", [c for c in WHOLE if "merge" not in c[4]],
+                         ids=[f"h{c[1]}d{c[3]}" for c in WHOLE if "merge" not in c[4]])
+def test_eight_waves_equal_four_over_the_line(oracle, torch_gpu, b, h, n, d, kw):
+    import spl_sage as S
+
+    p, q, k, v = _problem(oracle, b, h, n, d, kw, 200 + n)
+    _, base = run(torch_gpu, p, q, k, v, want_ws=False)
+    _, o = run(torch_gpu, p, q, k, v, want_ws=False, tile=S.Tile(8, 1, 3))
+    assert np.array_equal(o, base)
