@@ -351,8 +351,10 @@ public:
     // SageAttention::forward (mod.rs:888-900): prepare, then attend.
     void forward(Workspace& ws, const Tensor& q, const Tensor& k, const Tensor& v, const TensorMut& out,
                  const Options& opts = {}) const {
-        prepare(ws, q, k, v, opts);
-        attend(ws, out);
+        const sage_tensor tq = q.raw(), tk = k.raw(), tv = v.raw();
+        const sage_tensor_mut to = out.raw();
+        const sage_options o = opts.raw();
+        check(sage_forward(h_, ws.h_, &tq, &tk, &tv, &to, &o));
     }
 
     // forward without a workspace (sage_forward_noalloc; no counterpart in the

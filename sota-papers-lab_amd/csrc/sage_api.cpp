@@ -446,8 +446,9 @@ static sage_status check_tensor(const sage_strides& st, const void* data, uint64
 
 namespace sage {
 
-sage_status prepare_view(const sage_attention* s, const WsView& w, const sage_tensor* q, const sage_tensor* k,
-                         const sage_tensor* v, const sage_options* opts, Geom* geom, const QkvDev* qa) {
+// prepare's checks and kernel parameters.
+static sage_status prepare_geom(const sage_attention* s, const WsView& w, const sage_tensor* q, const sage_tensor* k,
+                                const sage_tensor* v, const sage_options* opts, Geom* geom) {
     const sage_plan& plan = w.plan;
     const uint64_t d = s->head_dim;
     const struct {
@@ -519,31 +520,91 @@ sage_status prepare_view(const sage_attention* s, const WsView& w, const sage_te
         g.dense_frames = (int)(l.dense_frames < l.frames ? l.dense_frames : l.frames);
     }
 
-    PrologueBufs bufs{w.q8, w.q_scale, w.k8, w.k_scale, w.v8, w.stats, w.part, w.kbias};
-    hipError_t e = launch_prologue((int)d, static_cast<const uint16_t*>(q->data), static_cast<const uint16_t*>(k->data),
-                                   static_cast<const uint16_t*>(v->data), opts->qk_norm_params, bufs, g, qa,
-                                   s->stream);
-    if (e != hipSuccess) return hip_fail(e, "launch sage prologue");
     *geom = g;
     return SAGE_OK;
 }
 
-sage_status attend_view(const sage_attention* s, const WsView& w, const Geom& geom, const sage_tensor_mut* out) {
-    const sage_plan& plan = w.plan;
-    sage_status r = check_tensor(out->strides, out->data, out->len, plan, plan.shape.heads, s->head_dim, "output");
+static sage_status launch_prepare(const sage_attention* s, const WsView& w, const sage_tensor* q, const sage_tensor* k,
+                                  const sage_tensor* v, const sage_options* opts, const Geom& g, const QkvDev* qa) {
+    PrologueBufs bufs{w.q8, w.q_scale, w.k8, w.k_scale, w.v8, w.stats, w.part, w.kbias};
+    hipError_t e = launch_prologue((int)s->head_dim, static_cast<const uint16_t*>(q->data),
+                                   static_cast<const uint16_t*>(k->data), static_cast<const uint16_t*>(v->data),
+                                   opts->qk_norm_params, bufs, g, qa, s->stream);
+    return e == hipSuccess ? SAGE_OK : hip_fail(e, "launch sage prologue");
+}
+
+sage_status prepare_view(const sage_attention* s, const WsView& w, const sage_tensor* q, const sage_tensor* k,
+                         const sage_tensor* v, const sage_options* opts, Geom* geom, const QkvDev* qa) {
+    Geom g;
+    sage_status r = prepare_geom(s, w, q, k, v, opts, &g);
+    if (r == SAGE_OK) r = launch_prepare(s, w, q, k, v, opts, g, qa);
+    if (r == SAGE_OK) *geom = g;
+    return r;
+}
+
+static sage_status attend_check(const sage_attention* s, const WsView& w, const sage_tensor_mut* out) {
+    sage_status r = check_tensor(out->strides, out->data, out->len, w.plan, w.plan.shape.heads, s->head_dim, "output");
     if (r != SAGE_OK) return r;
     if (out->dtype != SAGE_BF16 && out->dtype != SAGE_F16)
         return fail(SAGE_ERR_INVALID, "unknown dtype %d", out->dtype);
-    Geom g = geom;
+    return SAGE_OK;
+}
+
+// attend's kernel parameters and launch; q: the queries it quantises under
+// F_Q_LATER.
+static sage_status launch_attend(const sage_attention* s, const WsView& w, Geom g, const sage_tensor_mut* out,
+                                 const void* q) {
     g.o_sb = (long long)out->strides.batch;
     g.o_st = (long long)out->strides.token;
     g.o_sh = (long long)out->strides.head;
     g.flags = (g.flags & ~(F_OUT_F16 | F_WAVES8)) | (out->dtype == SAGE_F16 ? F_OUT_F16 : 0) |
               (s->config.tile.warps == 8 ? F_WAVES8 : 0);
-    AttendBufs bufs{w.q8, w.q_scale, w.k8, w.k_scale, w.v8, w.stats, w.kbias, out->data};
+    AttendBufs bufs{static_cast<const uint16_t*>(q), w.q8, w.q_scale, w.k8, w.k_scale, w.v8, w.stats, w.kbias, out->data};
     hipError_t e = launch_attention((int)s->head_dim, bufs, g, s->stream);
-    if (e != hipSuccess) return hip_fail(e, "launch sage attention");
-    return SAGE_OK;
+    return e == hipSuccess ? SAGE_OK : hip_fail(e, "launch sage attention");
+}
+
+sage_status attend_view(const sage_attention* s, const WsView& w, const Geom& geom, const sage_tensor_mut* out) {
+    sage_status r = attend_check(s, w, out);
+    return r == SAGE_OK ? launch_attend(s, w, geom, out, nullptr) : r;
+}
+
+// Whether the attention kernel may read Q while it writes `out`: it reads each
+// workgroup's query rows before it writes the same rows, so the two views are
+// the same or apart.
+static bool q_readable_beside(const sage_attention* s, const sage_plan& plan, const sage_tensor* q,
+                              const sage_tensor_mut* out) {
+    const sage_strides &a = q->strides, &b = out->strides;
+    if (q->data == out->data && a.batch == b.batch && a.token == b.token && a.head == b.head) return true;
+    const uint64_t nq = 2 * sage_strides_extent(&a, plan.shape.batch, plan.shape.tokens, plan.shape.heads, s->head_dim);
+    const uint64_t no = 2 * sage_strides_extent(&b, plan.shape.batch, plan.shape.tokens, plan.shape.heads, s->head_dim);
+    const uintptr_t pq = reinterpret_cast<uintptr_t>(q->data), po = reinterpret_cast<uintptr_t>(out->data);
+    return pq + nq <= po || po + no <= pq;
+}
+
+sage_status forward_view(const sage_attention* s, const WsView& w, const sage_tensor* q, const sage_tensor* k,
+                         const sage_tensor* v, const sage_options* opts, Geom* geom, const sage_tensor_mut* out,
+                         bool* prepared) {
+    Geom g;
+    sage_status r = prepare_geom(s, w, q, k, v, opts, &g);
+    if (r != SAGE_OK) return r;
+    // Queries are quantised by the attention kernel where it can and the
+    // output is one it will accept (otherwise prepare runs, then attend's
+    // refusal is reported, as for the two calls).
+    Geom probe = g;
+    if (s->config.tile.warps == 8) probe.flags |= F_WAVES8;
+    const bool later = attention_quantises_q((int)s->head_dim, probe) && attend_check(s, w, out) == SAGE_OK &&
+                       q_readable_beside(s, w.plan, q, out);
+    Geom run = g;
+    if (later) run.flags |= F_Q_LATER;
+    r = launch_prepare(s, w, q, k, v, opts, run, nullptr);
+    if (r != SAGE_OK) return r;
+    *geom = g;
+    *prepared = !later;
+    r = attend_check(s, w, out);
+    if (r == SAGE_OK) r = launch_attend(s, w, run, out, q->data);
+    if (r == SAGE_OK) *prepared = true;
+    return r;
 }
 
 }  // namespace sage
@@ -580,9 +641,16 @@ sage_status sage_attend(const sage_attention* s, const sage_workspace* ws, const
 
 sage_status sage_forward(const sage_attention* s, sage_workspace* ws, const sage_tensor* q, const sage_tensor* k,
                          const sage_tensor* v, const sage_tensor_mut* out, const sage_options* opts) {
-    sage_status r = sage_prepare(s, ws, q, k, v, opts);
-    if (r != SAGE_OK) return r;
-    return sage_attend(s, ws, out);
+    if (!out) {
+        sage_status r = sage_prepare(s, ws, q, k, v, opts);
+        return r == SAGE_OK ? sage_attend(s, ws, out) : r;
+    }
+    if (!s || !ws || !q || !k || !v || !opts) return fail(SAGE_ERR_INVALID, "null argument");
+    if (ws->head_dim != s->head_dim)
+        return fail(SAGE_ERR_INVALID, "workspace was made for head dim %llu, kernels are %llu", (u64)ws->head_dim,
+                    (u64)s->head_dim);
+    sage_status r = sage::forward_view(s, view_of(ws), q, k, v, opts, &ws->geom, out, &ws->prepared);
+    return r == SAGE_OK ? ok() : r;
 }
 
 }  // extern "C"

@@ -52,10 +52,125 @@
 
 namespace sage {
 
+// INT8 Q of a wave's 32 queries q0 .. q0 + 31 of one head (sage_quant.cu:85-127;
+// the prologue's tile_q8, the same codes and scales bit for bit), in a forward
+// call: the rows come from the 16-bit queries, the codes and scales go to the
+// workspace and, through `stage` (32 D bytes of LDS, this wave's alone), to
+// the wave's MFMA operands. Left to the prologue, Q costs it 2 bytes read and
+// one written an element, and one read back here, all at the memory's rate;
+// here the same bytes stream under the other workgroups' key loops, which
+// leave the memory idle. sage_prep at B2 H32 N4096 D128 41 -> 29 us, grouped
+// 32/8 N8192 27 -> 11; this kernel pays about 450 VALU instructions a wave and
+// the rows' latency, 8 us of 331. Whole forwards: 1.4 to 3.5% faster.
+// D/8 lanes hold a row, 8 channels a lane, 512/D rows at a time; rows past the
+// sequence are zeros. Its first half of iterations is the first 16-row group.
+template <int D>
+__device__ __forceinline__ void quantise_q(const uint16_t* __restrict__ q, int8_t* __restrict__ q8,
+                                           float* __restrict__ q_scale, const Geom& g, int q0, int lane,
+                                           uint8_t* stage, v4i (&qa)[D / 32], float& qs) {
+#pragma clang fp contract(off)
+    constexpr int CH = D / 8, RPI = 64 / CH, NI = 32 / RPI, KCPR = D / 16;
+    const int ch = lane % CH, slot = lane / CH;
+    typedef unsigned nt_u4 __attribute__((ext_vector_type(4)));
+    typedef unsigned nt_u2 __attribute__((ext_vector_type(2)));
+    nt_u4 raw[NI];
+    const uint16_t* row0 = q + (long long)(q0 + slot) * g.q_st + ch * 8;
+    const long long rstep = RPI * g.q_st;
+    if (q0 + 32 <= g.tokens) {
+#pragma unroll
+        for (int i = 0; i < NI; i++) raw[i] = __builtin_nontemporal_load(reinterpret_cast<const nt_u4*>(row0 + i * rstep));
+    } else {
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            raw[i] = nt_u4{0, 0, 0, 0};
+            if (q0 + slot + i * RPI < g.tokens)
+                raw[i] = __builtin_nontemporal_load(reinterpret_cast<const nt_u4*>(row0 + i * rstep));
+        }
+    }
+    // Row maxima on the 16-bit magnitudes, two a register: finite bf16 and
+    // fp16 magnitudes order like their bits, and anything above infinity's is
+    // a NaN, which fmaxf would skip (the general path below).
+    typedef unsigned short us2 __attribute__((ext_vector_type(2)));
+    const bool half = g.flags & F_IN_F16;
+    uint32_t top[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        us2 t = {0, 0};
+#pragma unroll
+        for (int i = j * NI / 2; i < (j + 1) * NI / 2; i++)
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                t = __builtin_elementwise_max(t, __builtin_bit_cast(us2, raw[i][c] & 0x7fff7fffu));
+        top[j] = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_max_u32(max((uint32_t)t.x, (uint32_t)t.y)));
+    }
+    float sc[2];
+    auto codes = [&](bool half, bool near, const float* amax) __attribute__((always_inline)) {
+        float inv[2];
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            inv[j] = amax[j] > 0.f ? 127.0f / amax[j] : 0.f;
+            sc[j] = amax[j] * (1.0f / 127.0f) * g.q_mul;
+        }
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            float x[8];
+            unpack8(make_uint4(raw[i].x, raw[i].y, raw[i].z, raw[i].w), x, half);
+            const float v = inv[2 * i / NI];
+#pragma unroll
+            for (int e = 0; e < 8; e++) x[e] = x[e] * v;
+            nt_u2 w;
+            w.x = near ? s8x4_near(x[0], x[1], x[2], x[3]) : s8x4(x[0], x[1], x[2], x[3]);
+            w.y = near ? s8x4_near(x[4], x[5], x[6], x[7]) : s8x4(x[4], x[5], x[6], x[7]);
+            const int row = slot + i * RPI;
+            __builtin_nontemporal_store(w, reinterpret_cast<nt_u2*>(q8 + row * D + ch * 8));
+            *reinterpret_cast<nt_u2*>(stage + 16 * swz(row * KCPR + (ch >> 1), KCPR) + 8 * (ch & 1)) = w;
+        }
+    };
+    // One branch on the input type and range for the whole tile.
+    float amax[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) amax[j] = half ? f16_to_f32(top[j]) : __uint_as_float(top[j] << 16);
+    const uint32_t inf = half ? 0x7c00u : 0x7f80u;
+    bool plain = true;  // no NaN, and 127 / amax finite (or no use made of it)
+#pragma unroll
+    for (int j = 0; j < 2; j++) plain = plain && top[j] <= inf && (top[j] == 0 || code_scale_ok(127.0f / amax[j]));
+    if (!plain) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            amax[j] = 0.f;
+            for (int i = j * NI / 2; i < (j + 1) * NI / 2; i++)
+                for (int c = 0; c < 4; c++) {
+                    const uint32_t w = raw[i][c];
+                    const float lo = half ? f16_to_f32(w & 0xffffu) : __uint_as_float(w << 16);
+                    const float hi = half ? f16_to_f32(w >> 16) : __uint_as_float(w & 0xffff0000u);
+                    amax[j] = fmaxf(amax[j], fmaxf(fabsf(lo), fabsf(hi)));
+                }
+            amax[j] = wave_max(amax[j]);
+        }
+        if (half)
+            codes(true, false, amax);
+        else
+            codes(false, false, amax);
+    } else if (half) {
+        codes(true, true, amax);
+    } else {
+        codes(false, true, amax);
+    }
+    if (lane < 2) q_scale[lane] = lane ? sc[1] : sc[0];
+    qs = lane & 16 ? sc[1] : sc[0];
+    // The wave's own LDS operations complete in order.
+#pragma unroll
+    for (int s = 0; s < D / 32; s++)
+        qa[s] = *reinterpret_cast<const v4i*>(stage + 16 * swz((lane & 31) * KCPR + 2 * s + (lane >> 5), KCPR));
+}
+
 // Workgroups a CU: four at head dim 64 (<= 128 VGPRs), three at head dim 128
 // (<= 168); the merged head-dim-128 kernel needs the registers of two.
-template <int D, bool CAUSAL, bool MERGE>
-__global__ __launch_bounds__(256, D == 64 ? 4 : (MERGE ? 2 : 3)) void sage_attn(const int8_t* __restrict__ q8, const float* __restrict__ q_scale,
+// QF (a forward call): the workgroup quantises its own queries (quantise_q)
+// instead of reading the prologue's codes.
+template <int D, bool CAUSAL, bool MERGE, bool QF>
+__global__ __launch_bounds__(256, D == 64 ? 4 : (MERGE ? 2 : 3)) void sage_attn(const uint16_t* __restrict__ q, int8_t* __restrict__ q8,
+                                                    float* __restrict__ q_scale,
                                                     const int8_t* __restrict__ k8,
                                                     const float* __restrict__ k_scale,
                                                     const uint8_t* __restrict__ v8, const float* __restrict__ stats,
@@ -105,25 +220,6 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : (MERGE ? 2 : 3)) void sage_attn(
     const int q0 = qt * ATTN_ROWS + wave * 32;  // first query of this wave
     const int qi = q0 + col;                    // this lane's query
 
-    // Q^T operand: lane holds channels 32s + 16*half .. +15 of its query.
-    v4i qa[KS];
-    {
-        const int8_t* qrow = q8 + (bh * g.tq_pad + qi) * D + 16 * half;
-#pragma unroll
-        for (int s = 0; s < KS; s++) qa[s] = *reinterpret_cast<const v4i*>(qrow + 32 * s);
-    }
-    // The Q scale; the key loop floors its product with the K scale (SCALE_FLOOR).
-    const float qs = q_scale[bh * (g.tq_pad / QGROUP) + (qi >> 4)];
-    // The Q scales of the wave's two 16-query groups (wave-uniform).
-    const float qsg0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(qs), 0));
-    const float qsg1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(qs), QGROUP));
-    // Consume the Q loads here, before the first barrier: otherwise the
-    // compiler sinks them into the key loop and waits for every outstanding
-    // load there, prefetches included.
-#pragma unroll
-    for (int s = 0; s < KS; s++) asm volatile("" ::"v"(qa[s]));
-    asm volatile("" ::"v"(qs));
-
     int nblk = g.kblocks;
     if (CAUSAL) nblk = min(nblk, (qt * ATTN_ROWS + ATTN_ROWS - 1) / BN + 1);
     // Leading blocks no query of the workgroup needs masked: every key exists
@@ -166,6 +262,37 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : (MERGE ? 2 : 3)) void sage_attn(
                                              (__attribute__((address_space(3))) void*)(dst + 16 * c0), 16, 0, 0);
         }
     };
+
+    // Q^T operand: lane holds channels 32s + 16*half .. +15 of its query.
+    v4i qa[KS];
+    // The Q scale; the key loop floors its product with the K scale (SCALE_FLOOR).
+    float qs;
+    if constexpr (QF) {
+        // The first tiles' copies fly meanwhile; the codes are staged in the
+        // other two buffers.
+        fetch(kg, 0, ldsK0, 0);
+        fetch(vg, 0, ldsV0, 1);
+        fetch_bias(0, ldsB0);
+        const int w2 = __builtin_amdgcn_readfirstlane(wave);
+        quantise_q<D>(q + b * g.q_sb + h * g.q_sh, q8 + (bh * g.tq_pad + q0) * D,
+                      q_scale + bh * (g.tq_pad / QGROUP) + q0 / QGROUP, g, q0, lane,
+                      (w2 < 2 ? ldsK1 : ldsV1) + (w2 & 1) * (TILE / 2), qa, qs);
+        __builtin_amdgcn_sched_barrier(0);
+    } else {
+        const int8_t* qrow = q8 + (bh * g.tq_pad + qi) * D + 16 * half;
+#pragma unroll
+        for (int s = 0; s < KS; s++) qa[s] = *reinterpret_cast<const v4i*>(qrow + 32 * s);
+        qs = q_scale[bh * (g.tq_pad / QGROUP) + (qi >> 4)];
+    }
+    // The Q scales of the wave's two 16-query groups (wave-uniform).
+    const float qsg0 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(qs), 0));
+    const float qsg1 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(qs), QGROUP));
+    // Consume the Q loads here, before the first barrier: otherwise the
+    // compiler sinks them into the key loop and waits for every outstanding
+    // load there, prefetches included.
+#pragma unroll
+    for (int s = 0; s < KS; s++) asm volatile("" ::"v"(qa[s]));
+    asm volatile("" ::"v"(qs));
 
     // Per-lane LDS byte offsets of the MFMA operands. K row 32t + col, chunk
     // 2ks + half sits at swz((32t + col) * KCPR + 2ks + half); 32t rows are a
@@ -428,9 +555,11 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : (MERGE ? 2 : 3)) void sage_attn(
         softmax_pv(blk, S0, v_cur, b_cur);
         __syncthreads();
     };
-    fetch(kg, 0, ldsK0, 0);
-    fetch(vg, 0, ldsV0, 1);
-    fetch_bias(0, ldsB0);
+    if constexpr (!QF) {
+        fetch(kg, 0, ldsK0, 0);
+        fetch(vg, 0, ldsV0, 1);
+        fetch_bias(0, ldsB0);
+    }
     __syncthreads();
     for (int blk = 0; blk < nblk; blk += 2) {
         step(blk, ldsK0, ldsK1, ldsV0, ldsV1, ldsB0, ldsB1);
@@ -760,18 +889,23 @@ static hipError_t launch_split(const AttendBufs& w, const Geom& g, hipStream_t s
 }
 #endif
 
+template <int D, bool CAUSAL, bool MERGE, bool QF>
+static hipError_t launch_q(const AttendBufs& w, const Geom& g, hipStream_t s) {
+    hipLaunchKernelGGL((sage_attn<D, CAUSAL, MERGE, QF>), dim3(g.tq_pad / ATTN_ROWS, g.heads, g.batch), dim3(256), 0, s,
+                       w.q, w.q8, w.q_scale, w.k8, w.k_scale, w.v8, w.stats, w.kbias, static_cast<uint16_t*>(w.out), g);
+    return hipGetLastError();
+}
+
 template <int D, bool CAUSAL, bool MERGE>
 static hipError_t launch_d(const AttendBufs& w, const Geom& g, hipStream_t s) {
-    hipLaunchKernelGGL((sage_attn<D, CAUSAL, MERGE>), dim3(g.tq_pad / ATTN_ROWS, g.heads, g.batch), dim3(256), 0, s,
-                       w.q8, w.q_scale, w.k8, w.k_scale, w.v8, w.stats, w.kbias, static_cast<uint16_t*>(w.out), g);
-    return hipGetLastError();
+    return g.flags & F_Q_LATER ? launch_q<D, CAUSAL, MERGE, true>(w, g, s) : launch_q<D, CAUSAL, MERGE, false>(w, g, s);
 }
 
 template <bool CAUSAL, bool MERGE>
 static hipError_t resources_of(int head_dim, int* regs, int* spill, int* lds) {
     hipFuncAttributes a;
-    const void* f = head_dim == 64 ? reinterpret_cast<const void*>(&sage_attn<64, CAUSAL, MERGE>)
-                                   : reinterpret_cast<const void*>(&sage_attn<128, CAUSAL, MERGE>);
+    const void* f = head_dim == 64 ? reinterpret_cast<const void*>(&sage_attn<64, CAUSAL, MERGE, false>)
+                                   : reinterpret_cast<const void*>(&sage_attn<128, CAUSAL, MERGE, false>);
     hipError_t e = hipFuncGetAttributes(&a, f);
     if (e != hipSuccess) return e;
     *regs = a.numRegs;
@@ -819,6 +953,12 @@ static int key_shares(int head_dim, const Geom& g) {
     }
     if (g.flags & F_CAUSAL) return n <= 208 ? 4 : n <= 320 ? 2 : 0;
     return n <= 160 ? 4 : 0;
+}
+
+// The whole-key four-wave kernels have the variant; the sage options' QK
+// LayerNorm of Q stays in the prologue.
+bool attention_quantises_q(int head_dim, const Geom& g) {
+    return !(g.flags & F_LN_Q) && (g.merge > 1 || !(g.flags & F_WAVES8)) && key_shares(head_dim, g) == 0;
 }
 
 // Dense, causal (an extension) or merged (sg_attn_merge); the API refuses

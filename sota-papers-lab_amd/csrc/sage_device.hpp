@@ -23,6 +23,7 @@ enum : int {
     F_IN_F16 = 32,
     F_OUT_F16 = 64,
     F_WAVES8 = 128,  // Tile { warps: 8 }: the eight-wave attention layout (dense and causal)
+    F_Q_LATER = 256,  // the attention kernel quantises Q (a forward call), not the prologue
 };
 
 // Kernel parameter block, passed by value. Element strides of the 16-bit
@@ -116,6 +117,21 @@ __device__ __forceinline__ uint32_t s8_code(float x) {
 __device__ __forceinline__ uint32_t s8x4(float a, float b, float c, float d) {
     return s8_code(a) | (s8_code(b) << 8) | (s8_code(c) << 16) | (s8_code(d) << 24);
 }
+
+// The same four codes for values of magnitude at most 127.5, or NaN: adding
+// 1.5 * 2^23 rounds each to the nearest even integer in the low mantissa bits
+// (a NaN's low byte is 0), so an add and three quarters of a byte permute a
+// value replace the round, convert, clamp, mask and shifts of s8x4. Quotients
+// x * (127 / amax) of |x| <= amax are such values wherever 127 / amax is
+// finite (code_scale_ok).
+__device__ __forceinline__ uint32_t s8x4_near(float a, float b, float c, float d) {
+    const float magic = 12582912.0f;
+    const uint32_t ua = __float_as_uint(a + magic), ub = __float_as_uint(b + magic);
+    const uint32_t uc = __float_as_uint(c + magic), ud = __float_as_uint(d + magic);
+    return __builtin_amdgcn_perm(ub, ua, 0x0c0c0400u) | __builtin_amdgcn_perm(ud, uc, 0x04000c0cu);
+}
+// inv = 127 / amax overflows for amax below 127 / FLT_MAX: its codes saturate.
+__device__ __forceinline__ bool code_scale_ok(float inv) { return inv <= 3.4028234663852886e38f; }
 
 // f32 -> E4M3 (OCP e4m3fn) codes of a (low byte) and b (high byte): round to
 // nearest even, saturating at +-448, NaN -> 0x7f, the semantics of
@@ -231,6 +247,33 @@ __device__ __forceinline__ float row_sum(float v) {
     if (CH > 4) v += dpp<0x141>(v);       // row_half_mirror: the other quad of the 8
     if (CH > 8) v += dpp<0x140>(v);       // row_mirror: the other 8 of the 16
     return v;
+}
+
+// Maximum over the wave's 64 lanes, in every lane, for values that are not
+// NaN: the rows of 16 by DPP as in row_sum, then the rows and the halves by
+// gfx950's lane swaps. Register moves only: the LDS crossbar's six shuffles
+// took a round trip each.
+__device__ __forceinline__ float wave_max(float v) {
+    v = fmaxf(v, dpp<0xB1>(v));
+    v = fmaxf(v, dpp<0x4E>(v));
+    v = fmaxf(v, dpp<0x141>(v));
+    v = fmaxf(v, dpp<0x140>(v));
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_int(v), __float_as_int(v), false, false);
+    v = fmaxf(__int_as_float((int)r[0]), __int_as_float((int)r[1]));
+    const auto h = __builtin_amdgcn_permlane32_swap(__float_as_int(v), __float_as_int(v), false, false);
+    return fmaxf(__int_as_float((int)h[0]), __int_as_float((int)h[1]));
+}
+
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+    auto step = [](uint32_t a, int b) __attribute__((always_inline)) { return a > (uint32_t)b ? a : (uint32_t)b; };
+    v = step(v, __builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xf, 0xf, false));
+    v = step(v, __builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xf, 0xf, false));
+    v = step(v, __builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xf, 0xf, false));
+    v = step(v, __builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xf, 0xf, false));
+    const auto r = __builtin_amdgcn_permlane16_swap((int)v, (int)v, false, false);
+    v = step((uint32_t)r[0], (int)r[1]);
+    const auto h = __builtin_amdgcn_permlane32_swap((int)v, (int)v, false, false);
+    return step((uint32_t)h[0], (int)h[1]);
 }
 
 struct QkvLane {

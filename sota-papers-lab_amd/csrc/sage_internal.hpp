@@ -32,10 +32,12 @@ struct PrologueBufs {
     float* kbias;  // [tk_pad]: log2 member count of each merged key, -inf past tk (merged plans)
 };
 
-// The attention kernel's inputs.
+// The attention kernel's inputs. Under F_Q_LATER q holds the 16-bit queries
+// and the kernel writes q8 and q_scale; otherwise it reads them (q is null).
 struct AttendBufs {
-    const int8_t* q8;
-    const float* q_scale;
+    const uint16_t* q;
+    int8_t* q8;
+    float* q_scale;
     const int8_t* k8;
     const float* k_scale;
     const uint8_t* v8;
@@ -66,6 +68,10 @@ hipError_t launch_attention_merged(int head_dim, const AttendBufs& w, const Geom
 // The keys-split kernels' launch, two or four shares of the keys a query
 // group (launch_attention calls it for grids of few query tiles).
 hipError_t launch_attention_keys(int head_dim, int shares, const AttendBufs& w, const Geom& g, hipStream_t s);
+
+// Whether a forward call on this geometry leaves Q's codes to the attention
+// kernel (F_Q_LATER).
+bool attention_quantises_q(int head_dim, const Geom& g);
 
 // Kernel resources (VGPRs, scratch, LDS) of the attention kernel for
 // head_dim: dense, causal or KV-merged; waves8 = the eight-wave layout that
@@ -115,5 +121,10 @@ sage_status workspace_layout(const sage_attention* s, const sage_shape* shape, c
 sage_status prepare_view(const sage_attention* s, const WsView& w, const sage_tensor* q, const sage_tensor* k,
                          const sage_tensor* v, const sage_options* opts, Geom* geom, const QkvDev* qa);
 sage_status attend_view(const sage_attention* s, const WsView& w, const Geom& geom, const sage_tensor_mut* out);
+// prepare_view then attend_view in one call: where the whole-key kernel runs,
+// Q's codes are left to it.
+sage_status forward_view(const sage_attention* s, const WsView& w, const sage_tensor* q, const sage_tensor* k,
+                         const sage_tensor* v, const sage_options* opts, Geom* geom, const sage_tensor_mut* out,
+                         bool* prepared);
 
 }  // namespace sage

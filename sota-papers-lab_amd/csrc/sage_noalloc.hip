@@ -105,9 +105,8 @@ extern "C" sage_status sage_forward_noalloc(const sage_attention* s, const sage_
                          static_cast<float*>(buf[6]),
                          static_cast<float*>(buf[7])};
     sage::Geom g;
-    st = sage::prepare_view(s, w, q, k, v, opts, &g, nullptr);
-    if (st != SAGE_OK) return st;
-    st = sage::attend_view(s, w, g, out);
+    bool prepared = false;
+    st = sage::forward_view(s, w, q, k, v, opts, &g, out, &prepared);
     if (st != SAGE_OK) return st;
     sage::set_error(SAGE_OK, "%s", "");
     return SAGE_OK;

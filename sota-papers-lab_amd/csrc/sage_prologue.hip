@@ -54,12 +54,6 @@ __device__ __forceinline__ void store16_once(void* p, uint4 w) {
     __builtin_nontemporal_store(nt_u4{w.x, w.y, w.z, w.w}, reinterpret_cast<nt_u4*>(p));
 }
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
-}
-
 // LayerNorm of one head row (sage_quant.cu:34-52) whose D channels lie on
 // D/8 consecutive lanes, 8 a lane (ch = lane's chunk); every lane of the wave
 // calls it. The lane sums meet in the reference's xor butterfly over
@@ -359,7 +353,8 @@ __device__ __forceinline__ void tile_q8(const uint16_t* __restrict__ q, const fl
 // INT8 Q of one query head of the KV head's group. The reference's one
 // thread block does all of it in turn; split, the streams of loads overlap
 // across workgroups, and grouped-query plans spread their Q heads over
-// workgroups instead of walking them in one.
+// workgroups instead of walking them in one. (F_Q_LATER: no Q roles, the
+// attention kernel quantises its own queries.)
 template <bool QKV>
 constexpr int stat_roles() { return QKV ? 2 : 1; }
 template <int D, bool LN, bool QKV>
@@ -372,7 +367,7 @@ __global__ __launch_bounds__(256) void sage_prep(const uint16_t* __restrict__ q,
     __shared__ float ginv[QTILE / QGROUP];
     __shared__ float red[8][4][D];
     constexpr int STATS = stat_roles<QKV>();
-    const int roles = STATS + g.group, tile = (int)blockIdx.x / roles, role = (int)blockIdx.x % roles;
+    const int roles = STATS + (g.flags & F_Q_LATER ? 0 : g.group), tile = (int)blockIdx.x / roles, role = (int)blockIdx.x % roles;
     const int hk = blockIdx.y, b = blockIdx.z;
     if (role >= STATS) {
         tile_q8<D, LN, QKV>(q, ln, q8, q_scale, g, qa, tile, hk, role - STATS, b, gmax, ginv);
@@ -836,7 +831,8 @@ hipError_t launch_qkv(int head_dim, const uint16_t* y, const QkvOutDev& o, const
 template <int D, bool LN, bool QKV>
 static hipError_t launch_prologue_d(const uint16_t* q, const uint16_t* k, const uint16_t* v, const float* ln,
                                     const PrologueBufs& w, const Geom& g, const QkvDev& qa, hipStream_t s) {
-    const long long prep_blocks = (long long)(stat_roles<QKV>() + g.group) * g.q_tiles;
+    const int q_roles = g.flags & F_Q_LATER ? 0 : g.group;
+    const long long prep_blocks = (long long)(stat_roles<QKV>() + q_roles) * g.q_tiles;
     if (prep_blocks > INT32_MAX) return hipErrorInvalidConfiguration;
     hipLaunchKernelGGL((sage_prep<D, LN, QKV>), dim3((unsigned)prep_blocks, g.kv_heads, g.batch), dim3(256), 0, s,
                        q, k, v, ln,

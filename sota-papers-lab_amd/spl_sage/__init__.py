@@ -487,8 +487,10 @@ class SageAttention:
 
     def forward(self, ws: Workspace, q: Tensor, k: Tensor, v: Tensor, out: TensorMut,
                 opts: Optional[Options] = None) -> None:
-        self.prepare(ws, q, k, v, opts)
-        self.attend(ws, out)
+        """prepare, then attend, as one call."""
+        o = (opts or Options())._c()
+        _check(lib().sage_forward(self._h, ws._h, C.byref(q._c()), C.byref(k._c()), C.byref(v._c()),
+                                  C.byref(out._c()), C.byref(o)))
 
     def prepare_qkv(self, ws: Workspace, input, norm=None, rope=None, opts: Optional[Options] = None) -> None:
         """prepare fed straight from the fused QKV projection (spl_sage.qkv)."""
