@@ -1,6 +1,6 @@
 // SageAttention2 prologue for gfx950: K/V channel statistics, INT8 Q (one
 // scale per 16 rows), INT8 K (one scale per 64 keys), FP8 E4M3 V (one scale
-// per channel). Three HBM-bound launches:
+// per channel). Three HBM-bound launches (two for short sequences):
 //
 //   sage_prep      grid ((1 + group) q_tiles, kv_heads, batch): per 128-token
 //                  tile, one workgroup writes the partial K sum, V sum, V min,
@@ -10,7 +10,8 @@
 //                  QKV projection, K and V get a workgroup each
 //                  ((2 + group) q_tiles)
 //   sage_finalize  grid (D / 4 channel groups of every KV head, dealt one
-//                  head an XCD): K mean, V mean, V scale, 1/V scale
+//                  head an XCD): K mean, V mean, V scale, 1/V scale (short
+//                  sequences: folded into sage_quant_kv instead)
 //   sage_quant_kv  grid (kblocks, kv_heads, batch): smoothed INT8 K and FP8 V,
 //                  V transposed per 64-key block into the MFMA operand order;
 //                  with KV merging each key pools its members (and the keys'
@@ -392,6 +393,71 @@ __global__ __launch_bounds__(256) void sage_prep(const uint16_t* __restrict__ q,
 // share every 128-byte line of its partials, so they are dealt to one XCD
 // (the dispatcher deals linear ids round-robin over the 8 XCDs): each line
 // then comes from HBM into one L2 once.
+// A channel's K sum, V sum, V min and V max to its K mean, V mean, V scale and
+// 1 / V scale.
+__device__ __forceinline__ void finish_stats(float* st, const Geom& g) {
+    const float n = (float)g.tokens;
+    const float mk = (g.flags & F_SMOOTH_K) ? st[0] / n : 0.f;
+    const float mv = (g.flags & F_SMOOTH_V) ? st[1] / n : 0.f;
+    const float amax = fmaxf(st[3] - mv, mv - st[2]);
+    st[0] = mk;
+    st[1] = mv;
+    st[2] = amax > 0.f ? amax / g.v_range : 1.0f;
+    st[3] = 1.0f / st[2];
+}
+
+// The same fold inside every sage_quant_kv workgroup, for sequences of few
+// tiles: it saves a launch (about 2.5 us of the host's time and 2 to 4 of the
+// GPU's), and costs each workgroup its head's partials, q_tiles / 16 of the K
+// and V bytes it reads anyway, from L2. Whole prologue, us, three launches /
+// folded: D 64 H 2 N 256 10.4 / 8.7, H 16 N 689 11.5 / 10.0, B 8 H 16 N 689
+// 24.9 / 22.3, H 16 N 2048 (16 tiles) 13.4 / 11.9, B 8 H 16 N 2048 44.7 / 44.8,
+// N 2756 (22) 56.1 / 59.3; D 128 H 32 N 1000 18.1 / 16.7, B 8 H 16 N 1378 (11)
+// 59.5 / 58.0, H 16 N 2048 (16) 17.6 / 18.3, B 8 N 2756 103.9 / 109.3. So up to
+// 16 tiles at head dim 64 and 12 at 128 (two columns a thread).
+//
+// One thread a (statistic, channel) column, its loads independent, in
+// sage_finalize's order (even and odd tiles apart). `out` receives the four
+// statistics of the head's channels; the first workgroup of a head stores them.
+constexpr int FOLD_TILES_64 = 16, FOLD_TILES_128 = 12;
+template <int D>
+__device__ __forceinline__ void fold_tiles(const float* __restrict__ part, float* __restrict__ stats, const Geom& g,
+                                           bool store, float* out) {
+#pragma unroll
+    for (int c = threadIdx.x; c < 4 * D; c += 256) {
+        const int stat = c / D;  // wave-uniform
+        float r[2];
+        r[0] = r[1] = stat < 2 ? 0.f : (stat == 2 ? 3.0e38f : -3.0e38f);
+        auto fold = [&](auto op) __attribute__((always_inline)) {
+#pragma unroll 4
+            for (int t = 0; t + 1 < g.q_tiles; t += 2) {
+                r[0] = op(r[0], part[(long long)t * 4 * D + c]);
+                r[1] = op(r[1], part[(long long)(t + 1) * 4 * D + c]);
+            }
+            if (g.q_tiles & 1) r[0] = op(r[0], part[(long long)(g.q_tiles - 1) * 4 * D + c]);
+            out[c] = op(r[0], r[1]);
+        };
+        if (stat < 2)
+            fold([](float a, float b) { return a + b; });
+        else if (stat == 2)
+            fold([](float a, float b) { return fminf(a, b); });
+        else
+            fold([](float a, float b) { return fmaxf(a, b); });
+    }
+    __syncthreads();
+    if (threadIdx.x < D) {
+        const int d = threadIdx.x;
+        float st[4] = {out[d], out[D + d], out[2 * D + d], out[3 * D + d]};
+        finish_stats(st, g);
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            out[s * D + d] = st[s];
+            if (store) stats[s * D + d] = st[s];
+        }
+    }
+    __syncthreads();
+}
+
 constexpr int FIN_CH = 4;
 constexpr int FIN_CHUNK = 512;
 template <int D>
@@ -466,16 +532,10 @@ __global__ __launch_bounds__(256) void sage_finalize(const float* __restrict__ p
             const float r0 = fin[s2][0][c], r1 = fin[s2][1][c];
             st[s2] = s2 < 2 ? r0 + r1 : (s2 == 2 ? fminf(r0, r1) : fmaxf(r0, r1));
         }
-        const float n = (float)g.tokens;
-        const float mk = (g.flags & F_SMOOTH_K) ? st[0] / n : 0.f;
-        const float mv = (g.flags & F_SMOOTH_V) ? st[1] / n : 0.f;
-        const float amax = fmaxf(st[3] - mv, mv - st[2]);
-        const float scale = amax > 0.f ? amax / g.v_range : 1.0f;
+        finish_stats(st, g);
         float* o = stats + bhk * 4 * D;
-        o[d] = mk;
-        o[D + d] = mv;
-        o[2 * D + d] = scale;
-        o[3 * D + d] = 1.0f / scale;
+#pragma unroll
+        for (int s2 = 0; s2 < 4; s2++) o[s2 * D + d] = st[s2];
     }
 }
 
@@ -504,9 +564,10 @@ __device__ __forceinline__ void put_v(uint8_t* vt, int ch, int kl, const float* 
 template <int D, bool LN, bool QKV>
 __global__ __launch_bounds__(256) void sage_quant_kv(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
                                                      const float* __restrict__ ln,
-                                                     const float* __restrict__ stats, int8_t* __restrict__ k8,
+                                                     float* __restrict__ stats, int8_t* __restrict__ k8,
                                                      float* __restrict__ k_scale, uint8_t* __restrict__ v8,
-                                                     float* __restrict__ kbias, Geom g, QkvDev qa) {
+                                                     float* __restrict__ kbias, const float* __restrict__ part,
+                                                     Geom g, QkvDev qa) {
     constexpr int CH = D / 8;
     constexpr int TPI = 256 / CH;
     constexpr int NI = KBLOCK / TPI;
@@ -517,15 +578,26 @@ __global__ __launch_bounds__(256) void sage_quant_kv(const uint16_t* __restrict_
 
     __shared__ unsigned kmax;
     __shared__ __attribute__((aligned(16))) uint8_t vt[D * KBLOCK];
+    __shared__ float fold[4 * D];
     if (tid == 0) kmax = 0u;
 
     const float* st = stats + bhk * 4 * D;
     float mk[8], mv[8], iv[8];
+    if (part) {
+        fold_tiles<D>(part + bhk * g.q_tiles * 4 * D, stats + bhk * 4 * D, g, blk == 0, fold);
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-        mk[e] = st[ch * 8 + e];
-        mv[e] = st[D + ch * 8 + e];
-        iv[e] = st[3 * D + ch * 8 + e];
+        for (int e = 0; e < 8; e++) {
+            mk[e] = fold[ch * 8 + e];
+            mv[e] = fold[D + ch * 8 + e];
+            iv[e] = fold[3 * D + ch * 8 + e];
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            mk[e] = st[ch * 8 + e];
+            mv[e] = st[D + ch * 8 + e];
+            iv[e] = st[3 * D + ch * 8 + e];
+        }
     }
     float kv[NI][8];
     float amax = 0.f;
@@ -839,13 +911,16 @@ static hipError_t launch_prologue_d(const uint16_t* q, const uint16_t* k, const 
                        w.q8, w.q_scale, w.part, w.k8, w.v8, g, qa);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const long long heads8 = ((long long)g.batch * g.kv_heads + NUM_XCD - 1) / NUM_XCD * NUM_XCD;
-    if (heads8 * (D / FIN_CH) > INT32_MAX) return hipErrorInvalidConfiguration;
-    hipLaunchKernelGGL(sage_finalize<D>, dim3((unsigned)(heads8 * (D / FIN_CH))), dim3(256), 0, s, w.part, w.stats, g);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
+    const bool fold = g.q_tiles <= (D == 64 ? FOLD_TILES_64 : FOLD_TILES_128);
+    if (!fold) {
+        const long long heads8 = ((long long)g.batch * g.kv_heads + NUM_XCD - 1) / NUM_XCD * NUM_XCD;
+        if (heads8 * (D / FIN_CH) > INT32_MAX) return hipErrorInvalidConfiguration;
+        hipLaunchKernelGGL(sage_finalize<D>, dim3((unsigned)(heads8 * (D / FIN_CH))), dim3(256), 0, s, w.part, w.stats, g);
+        e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
     hipLaunchKernelGGL((sage_quant_kv<D, LN, QKV>), dim3(g.kblocks, g.kv_heads, g.batch), dim3(256), 0, s, k, v, ln,
-                       w.stats, w.k8, w.k_scale, w.v8, w.kbias, g, qa);
+                       w.stats, w.k8, w.k_scale, w.v8, w.kbias, fold ? w.part : nullptr, g, qa);
     return hipGetLastError();
 }
 
