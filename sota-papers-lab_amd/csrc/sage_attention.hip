@@ -921,50 +921,66 @@ static hipError_t resources_of(int head_dim, int* regs, int* spill, int* lds) {
 // default order and are built in the second pass.
 #ifndef SAGE_ATTN_MERGED
 
-// How many shares the keys of a query group are split into (sage_attn_keys),
-// or 0 for the whole-key kernels, by the number of 128-query tiles: n / 256 a
-// CU. A tile is one wave a SIMD, and a lone wave takes 1.6 times the chip's
-// best time a block, so up to n = 256 the chip is short of waves however long
-// the keys; a split has more of them but reads K and V once per 32 or 64
-// queries instead of 128 and sweeps the keys' first shares twice (15 to 20%
-// slower at head dim 64 on a full chip, 30 to 35% at 128, where its LDS holds
-// two waves a SIMD). Measured (us, whole keys / four shares / two):
+// How the keys are split (KeySplit), by the number n of 128-query tiles and
+// their remainder r over whole multiples of the chip's 256 CUs.
+//
+// Few tiles. A tile is one wave a SIMD, and a lone wave takes 1.6 times the
+// chip's best time a block, so up to about n = 256 the chip is short of waves
+// however long the keys; four or two shares make more of them, but read K and V
+// once per 32 queries instead of 128 and sweep the keys' first shares twice (20
+// to 35% slower on a full chip). Measured (us, whole keys / four / two shares):
 //   D 64        96 tiles N 689: 11.8 / 8.0 / 9.1     176, N 1378: 19.9 / 16.7 / 19.0
-//               256, N 1000: 16.7 / 16.3 / 15.9      352, N 2756: 52.5 / 48.1 / 46.3
-//               384, N 2048: 40.7 / 38.6 / 36.4      480, N 5000: 92.1 / 104 / 95.2
+//               216, N 1100: 18.2 / 17.9             256, N 1000: 17.3 / 17.2 / 17.1
 //   D 64 causal 256, N 1000: 16.3 / 11.5 / 12.9      352, N 2756: 36.2 / 27.6 / 28.6
 //               480, N 5000: 81.3 / 67.8 / 63.2      704, N 5512: 78.5 / 84.5 / 79.8
 //   D 128       128, N 8192: 118 / 76.9 / 84.7       176, N 1378: 27.6 / 27.5 / 27.8
-//               256, N 1000: 23.2 / 28.5 / 24.1
 //   D 128 causal 176, N 1378: 26.8 / 20.7 / 21.2     256, N 1000: 22.3 / 21.5 / 18.9
 //               352, N 2756: 49.3 / 47.7 / 43.9      384, N 689: 18.0 / 24.5 / 21.8
 //   merged      D 64 96 tiles, stride 2: 7.2 / 6.2 / 6.4, stride 4: 5.5 / 5.7 / 5.3;
 //               D 128 96, stride 2: 9.8 / 8.6 / 8.7, stride 4: 8.2 / 8.2 / 7.1;
 //               352 D 64: 21.9 / 23.4 / 21.9, D 128: 29.8 / 41.5 / 37.9
 // (A causal tile's keys end at its queries, so causal grids carry half the
-// work and longer tails. The tile of the context's Config does not matter
-// here: it picks a layout, never a result.)
-static int key_shares(int head_dim, const Geom& g) {
+// work and longer tails.)
+//
+// A few tiles over. Whole tiles alone give r CUs one tile more than the rest,
+// and those set the time. Left whole beside the others split into four
+// workgroups each, the remainder spreads over all CUs (us, all whole / r split):
+//   D 64  r 8 over 256, N 1000: 23.3 / 17.0   96, N 2756: 52.5 / 37.4   128, N 2048: 38.8 / 29.8
+//         186, N 4300: 79.1 / 72.8            224, N 5000: 85.1 / 90.5
+//         44 over 512, N 17776: 354 / 293     128, N 1000: 31.8 / 27.6  160, N 1000: 31.6 / 31.7
+//         64 over 768, N 1000: 39.1 / 34.6    123, N 12600: 334 / 303
+//         74 over 1024, N 15500: 498 / 447    84 over 1280, N 15800: 597 / 568   64 over 1536: 66.9 / 61.9
+//   D 128 8 over 256, N 1000: 30.9 / 25.5     96, N 2756: 63.5 / 59.8   128, N 2048: 50.9 / 49.9
+//         44 over 512, N 17776: 483 / 423     64, N 1000: 44.9 / 39.0   96, N 1000: 45.2 / 45.2
+//         64 over 768, N 1000: 59.8 / 52.3    74 over 1024, N 15500: 690 / 672   16 over 1280: 82.6 / 76.3
+// (A forward call's Q codes cost 2% more outside sage_attn, so gains below
+// that are left.) The tile of the context's Config does not matter here: it
+// picks a layout, never a result.
+static KeySplit key_split(int head_dim, const Geom& g) {
     const long long n = (long long)g.q_tiles * g.heads * g.batch;
-    if (g.merge > 1) return n <= (head_dim == 64 ? 224 : 128) ? 2 : 0;
-    if (head_dim == 64) {
-        if (g.flags & F_CAUSAL) return n <= 320 ? 4 : n <= 560 ? 2 : 0;
-        return n <= 224 ? 4 : n <= 416 ? 2 : 0;
+    if (g.merge > 1) return {n <= (head_dim == 64 ? 224 : 128) ? 2 : 0, 0};
+    if (g.flags & F_CAUSAL) {
+        if (head_dim == 64) return {n <= 320 ? 4 : n <= 560 ? 2 : 0, 0};
+        return {n <= 208 ? 4 : n <= 320 ? 2 : 0, 0};
     }
-    if (g.flags & F_CAUSAL) return n <= 208 ? 4 : n <= 320 ? 2 : 0;
-    return n <= 160 ? 4 : 0;
+    if (n <= (head_dim == 64 ? 224 : 160)) return {4, 0};
+    // The largest remainder that is split beside 1, 2, .. tiles a CU.
+    static constexpr int MOST[2][6] = {{176, 136, 112, 80, 80, 64}, {96, 72, 80, 48, 32, 0}};
+    const long long f = n / 256, r = n % 256;
+    if (f >= 1 && f <= 6 && r > 0 && r <= MOST[head_dim == 128][f - 1]) return {4, (int)(n - r)};
+    return {0, 0};
 }
 
 // The whole-key four-wave kernels have the variant; the sage options' QK
 // LayerNorm of Q stays in the prologue.
 bool attention_quantises_q(int head_dim, const Geom& g) {
-    return !(g.flags & F_LN_Q) && (g.merge > 1 || !(g.flags & F_WAVES8)) && key_shares(head_dim, g) == 0;
+    return !(g.flags & F_LN_Q) && (g.merge > 1 || !(g.flags & F_WAVES8)) && key_split(head_dim, g).shares == 0;
 }
 
 // Dense, causal (an extension) or merged (sg_attn_merge); the API refuses
 // causal masking over merged keys.
 hipError_t launch_attention(int head_dim, const AttendBufs& w, const Geom& g, hipStream_t s) {
-    if (const int shares = key_shares(head_dim, g)) return launch_attention_keys(head_dim, shares, w, g, s);
+    if (const KeySplit k = key_split(head_dim, g); k.shares) return launch_attention_keys(head_dim, k, w, g, s);
     if (g.merge > 1) return launch_attention_merged(head_dim, w, g, s);
     if (g.flags & F_WAVES8) {
         if (head_dim == 64)

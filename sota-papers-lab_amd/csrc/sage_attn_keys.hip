@@ -7,9 +7,12 @@
 // chain (0.66 us a block at head dim 64, 1.6 times the chip's best rate). Here
 // S = 4 or 2 waves share 32 queries, each taking a 1/S share of their key
 // blocks: S times as many waves, each with 1/S of the chain. A workgroup is
-// four waves: one query group under S = 4, two under S = 2. key_shares
-// (sage_attention.hip) says which grids run here and what both sides measured:
-// 96 tiles of 689 keys 11.8 -> 8.0 us, 128 of 8192 at head dim 128 118 -> 77.
+// four waves: one query group under S = 4, two under S = 2. The HET variant
+// (dense, S = 4) leaves most 128-query tiles whole, one workgroup each as in
+// sage_attn, and splits the few over a whole number a CU, so that these spread
+// over all CUs. key_split (sage_attention.hip) says which grids run here and
+// what both sides measured: 96 tiles of 689 keys 11.8 -> 8.0 us, 128 of 8192 at
+// head dim 128 118 -> 77, 352 of 2756 52.5 -> 37.4.
 //
 // The arithmetic is the reference's online softmax (sezer-muhammed/
 // sota-papers-lab, platform/spl-nn/cuda/sage_attn.cu:135-424) with its running
@@ -25,8 +28,10 @@
 // reading K and V once per 32 queries. One K and one V buffer suffice: K(j + 1)
 // is fetched over K(j) once QK^T has read it and lands during the softmax and
 // P.V; V(j + 1) over V(j) after P.V, landing during the next QK^T and softmax.
-// Four workgroups a CU at head dim 64 (registers), two at 128 (LDS; one
-// buffer for both tiles and three workgroups measured no better).
+// Four workgroups a CU at head dim 64 (registers), two at 128 (LDS). HET at
+// head dim 128 takes one buffer a wave for both tiles (ONE: V(j) over K(j), K(j
+// + 1) over V(j), their latency left to the other waves), three workgroups a
+// CU: its whole tiles fill the chip and want the waves.
 #include "sage_attn_device.hpp"
 #include "sage_internal.hpp"
 
@@ -61,6 +66,16 @@ __device__ __forceinline__ void copy_4k(const uint8_t* base, uint32_t even, uint
         : "memory");
 #endif
 }
+// 1 KB, 16 bytes a lane.
+__device__ __forceinline__ void copy_1k(const uint8_t* base, uint32_t off, uint32_t dst) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile(
+        "s_mov_b32 m0, %0\n\t"
+        "s_nop 0\n\t"
+        "global_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane((int)dst)), "v"(off), "s"(base)
+        : "memory");
+#endif
+}
 // 256 bytes, four a lane.
 __device__ __forceinline__ void copy_256(const uint8_t* base, uint32_t off, uint32_t dst) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -85,15 +100,42 @@ __device__ __forceinline__ void wait_reads() {
 #endif
 }
 
-template <int D, bool CAUSAL, bool MERGE, int S>
-__global__ __launch_bounds__(256, D == 64 ? (MERGE ? 3 : 4) : 2) void sage_attn_keys(
+// The workgroup's LDS accesses so far are done; copies may still fly.
+__device__ __forceinline__ void block_barrier() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#endif
+}
+__device__ __forceinline__ void store4(uint16_t* p, const float* y, bool f16) {
+    uint2 w;
+    if (f16) {
+        w.x = pack_f16x2(y[0], y[1]);
+        w.y = pack_f16x2(y[2], y[3]);
+    } else {
+        w.x = pack_bf16x2(y[0], y[1]);
+        w.y = pack_bf16x2(y[2], y[3]);
+    }
+    *reinterpret_cast<uint2*>(p) = w;
+}
+
+// The grid of whole tiles beside split ones: 128-query tiles, dealt to the XCDs
+// in contiguous ranges, of which an XCD's first whole8 are one workgroup each
+// and the others four.
+struct KeyGrid {
+    int tiles, whole8;
+};
+
+template <int D, bool CAUSAL, bool MERGE, int S, bool HET>
+__global__ __launch_bounds__(256, D == 64 ? (MERGE ? 3 : 4) : (HET ? 3 : 2)) void sage_attn_keys(
     const int8_t* __restrict__ q8, const float* __restrict__ q_scale, const int8_t* __restrict__ k8,
     const float* __restrict__ k_scale, const uint8_t* __restrict__ v8, const float* __restrict__ stats,
-    const float* __restrict__ kbias, uint16_t* __restrict__ out, Geom g) {
+    const float* __restrict__ kbias, uint16_t* __restrict__ out, Geom g, KeyGrid kg8) {
     constexpr int BN = ATTN_BN, KS = D / 32, DT = D / 32, TILE = BN * D, KCPR = D / 16;
     constexpr int NL = TILE / 1024;  // 1 KB copies a tile
+    constexpr bool ONE = HET && D == 128;
     __shared__ __attribute__((aligned(16))) uint8_t ldsK[KEY_WAVES * TILE];
-    __shared__ __attribute__((aligned(16))) uint8_t ldsV[KEY_WAVES * TILE];
+    __shared__ __attribute__((aligned(16))) uint8_t ldsV2[ONE ? 16 : KEY_WAVES * TILE];
+    uint8_t* const ldsV = ONE ? ldsK : ldsV2;
     // The first sweep's maxima before shares 1 .. S - 1, [share - 1][wave][lane].
     __shared__ float ldsM[(S - 1) * KEY_WAVES * 64];
     __shared__ float ldsE[KEY_WAVES * 64];  // the running maximum after a share, [wave][lane]
@@ -105,27 +147,51 @@ __global__ __launch_bounds__(256, D == 64 ? (MERGE ? 3 : 4) : 2) void sage_attn_
 
     const int tid = threadIdx.x, lane = tid & 63, col = lane & 31, half = lane >> 5;
     const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int ntq = gridDim.x;
-    const int lin = blockIdx.x + ntq * (blockIdx.y + gridDim.y * blockIdx.z), total = ntq * gridDim.y * gridDim.z;
-    int qt, hb;  // query tile; head slot b * heads + h (dealt as sage_attn deals its tiles)
-    if (CAUSAL && causal_longest_first(total, ntq)) {
-        const int per = total / NUM_XCD, hx = per / ntq, x = lin % NUM_XCD, i = lin / NUM_XCD;
-        qt = ntq - 1 - i / hx;
-        hb = x * hx + i % hx;
+    static_assert(!HET || (S == 4 && !CAUSAL && !MERGE), "whole tiles beside four shares: dense plans");
+    int qt, hb;  // query tile; head slot b * heads + h
+    int grp, part, q0;
+    bool whole = false;
+    if constexpr (HET) {
+        // XCD x holds tiles [x n / 8, (x + 1) n / 8).
+        const int lin = blockIdx.x, x = lin % NUM_XCD, i = lin / NUM_XCD;
+        const int t0 = (int)((long long)x * kg8.tiles / NUM_XCD), cnt = (int)((long long)(x + 1) * kg8.tiles / NUM_XCD) - t0;
+        const int ntq = g.q_tiles;
+        whole = i < kg8.whole8;
+        const int t = whole ? i : kg8.whole8 + (i - kg8.whole8) / 4, sub = (i - kg8.whole8) % 4;
+        if (t >= cnt) return;
+        qt = (t0 + t) % ntq;
+        hb = (t0 + t) / ntq;
+        grp = 0;
+        part = wv;
+        q0 = 128 * qt + 32 * (whole ? wv : sub);
+        if (!whole && q0 >= g.tokens) return;
     } else {
-        const int tile = xcd_tile(lin, total);
-        qt = CAUSAL ? ntq - 1 - tile % ntq : tile % ntq;
-        hb = tile / ntq;
+        const int ntq = gridDim.x;
+        const int lin = blockIdx.x + ntq * (blockIdx.y + gridDim.y * blockIdx.z), total = ntq * gridDim.y * gridDim.z;
+        if (CAUSAL && causal_longest_first(total, ntq)) {
+            const int per = total / NUM_XCD, hx = per / ntq, x = lin % NUM_XCD, i = lin / NUM_XCD;
+            qt = ntq - 1 - i / hx;
+            hb = x * hx + i % hx;
+        } else {
+            const int tile = xcd_tile(lin, total);
+            qt = CAUSAL ? ntq - 1 - tile % ntq : tile % ntq;
+            hb = tile / ntq;
+        }
+        grp = wv / S;
+        part = wv % S;
+        q0 = qt * (KEY_WAVES / S * KEY_ROWS) + grp * KEY_ROWS;
     }
     const int h = hb % g.heads, b = hb / g.heads, hk = h / g.group;
     const long long bh = (long long)b * g.heads + h, bhk = (long long)b * g.kv_heads + hk;
-    const int grp = wv / S, part = wv % S;  // query group in the workgroup; key share
-    const int q0 = qt * (KEY_WAVES / S * KEY_ROWS) + grp * KEY_ROWS, qi = q0 + col;
+    const int qi = q0 + col;
 
+    // Blocks this wave's group (a whole tile: the workgroup) attends, and
+    // those of them that no query needs masked.
+    const int qlo = HET && whole ? 128 * qt : q0, qhi = HET && whole ? 128 * qt + 127 : q0 + KEY_ROWS - 1;
     int nblk = g.kblocks;
-    if (CAUSAL) nblk = min(nblk, (q0 + KEY_ROWS - 1) / BN + 1);
+    if (CAUSAL) nblk = min(nblk, qhi / BN + 1);
     int nfull = MERGE ? nblk : min(nblk, g.tk / BN);
-    if (CAUSAL) nfull = min(nfull, (q0 + 1) / BN);
+    if (CAUSAL) nfull = min(nfull, (qlo + 1) / BN);
     // This wave's blocks (none where nblk < S and part is small).
     const int lo = part * nblk / S, hi = (part + 1) * nblk / S;
 
@@ -192,17 +258,21 @@ __global__ __launch_bounds__(256, D == 64 ? (MERGE ? 3 : 4) : 2) void sage_attn_
     auto qk = [&](const uint8_t* kp, v16i (&s)[2]) __attribute__((always_inline)) {
         uint4 ka[2][KS];
 #pragma unroll
-        for (int t = 0; t < 2; t++)
+        for (int t = 0; t < 2; t++) {
 #pragma unroll
             for (int ks = 0; ks < KS; ks++)
                 ka[t][ks] = *reinterpret_cast<const uint4*>(kp + 16 * 32 * t * KCPR + koff[ks]);
+            // (Three waves a SIMD at head dim 128: one sub-tile's operands at a time.)
+            if (!ONE && t == 0) continue;
 #pragma unroll
-        for (int t = 0; t < 2; t++)
+            for (int u = ONE ? t : 0; u <= t; u++)
 #pragma unroll
-            for (int ks = 0; ks < KS; ks++) {
-                const v4i av = {(int)ka[t][ks].x, (int)ka[t][ks].y, (int)ka[t][ks].z, (int)ka[t][ks].w};
-                s[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, qa[ks], ks ? s[t] : magic, 0, 0, 0);
-            }
+                for (int ks = 0; ks < KS; ks++) {
+                    const v4i av = {(int)ka[u][ks].x, (int)ka[u][ks].y, (int)ka[u][ks].z, (int)ka[u][ks].w};
+                    s[u] = __builtin_amdgcn_mfma_i32_32x32x32_i8(av, qa[ks], ks ? s[u] : magic, 0, 0, 0);
+                }
+            if (ONE && t == 0) __builtin_amdgcn_sched_barrier(0);
+        }
     };
     // The block's logit scale; masked blocks set scores past the sequence (or
     // the query) to -inf and floor it (SCALE_FLOOR).
@@ -272,7 +342,27 @@ __global__ __launch_bounds__(256, D == 64 ? (MERGE ? 3 : 4) : 2) void sage_attn_
     float mp[S - 1];
 #pragma unroll
     for (int i = 0; i < S - 1; i++) mp[i] = -1.0e30f;
-    {
+    if constexpr (ONE) {
+        auto fetch1 = [&](int blk) __attribute__((always_inline)) {
+            if (blk < pre) fetch(kg, blk, kdst, true);
+        };
+        if (!whole) {
+            fetch1(part);
+            for (int blk = part; blk < pre; blk += S) {
+                const float kscf = k_scale_of(blk);
+                wait_copies<0>();
+                v16i s0[2];
+                qk(kt, s0);
+                wait_reads();
+                fetch1(blk + S);
+                const float scl = scale_mask(blk, kscf, s0);
+                const float r = row_max(s0, scl, x);
+#pragma unroll
+                for (int i = 0; i < S - 1; i++)
+                    if (blk < (i + 1) * nblk / S) mp[i] = running_max(mp[i], r);
+            }
+        }
+    } else if (!whole) {
         auto fetch2 = [&](int blk) __attribute__((always_inline)) {
             if (blk < pre) {
                 fetch_bias(blk, 0);
@@ -320,17 +410,19 @@ __global__ __launch_bounds__(256, D == 64 ? (MERGE ? 3 : 4) : 2) void sage_attn_
             }
         }
     }
-    fetch_bias(first, first & 1);
-    fetch(kg, first, kdst, true);
-    fetch(vg, first, vdst, false);
-#pragma unroll
-    for (int i = 0; i < S - 1; i++) ldsM[(i * KEY_WAVES + wv) * 64 + lane] = mp[i];
-    __syncthreads();
-    // The running maximum before this wave's first block.
     float m = -1.0e30f;
-    if (part > 0) {
+    if (!whole) {
+        fetch_bias(first, first & 1);
+        fetch(kg, first, kdst, true);
+        if (!ONE) fetch(vg, first, vdst, false);
 #pragma unroll
-        for (int i = 0; i < S; i++) m = running_max(m, ldsM[((part - 1) * KEY_WAVES + grp * S + i) * 64 + lane]);
+        for (int i = 0; i < S - 1; i++) ldsM[(i * KEY_WAVES + wv) * 64 + lane] = mp[i];
+        __syncthreads();
+        // The running maximum before this wave's first block.
+        if (part > 0) {
+#pragma unroll
+            for (int i = 0; i < S; i++) m = running_max(m, ldsM[((part - 1) * KEY_WAVES + grp * S + i) * 64 + lane]);
+        }
     }
 
     v16i sc[2];
@@ -341,12 +433,14 @@ __global__ __launch_bounds__(256, D == 64 ? (MERGE ? 3 : 4) : 2) void sage_attn_
         for (int r = 0; r < 16; r++) o[dt][r] = 0.f;
     float l = 0.f;
     v8i pb = {};
-    auto step = [&](int blk, bool more) __attribute__((always_inline)) {
-        wait_copies<NL>();  // K(blk) (and its bias) are in; V(blk)'s copies may still fly
-        qk(kt, sc);
-        wait_reads();
+    auto step = [&](int blk, bool more, bool shared, const uint8_t* kp, const uint8_t* vp)
+                    __attribute__((always_inline)) {
+        if (!shared) wait_copies<ONE ? 0 : NL>();  // K(blk) (and its bias) are in; V(blk)'s copies may still fly
+        qk(kp, sc);
+        if (!shared) wait_reads();
         const float kscf = k_scale_of(blk);
-        if (more) {
+        if (!shared && ONE) fetch(vg, blk, kdst, false);
+        if (!shared && more && !ONE) {
             fetch_bias(blk + 1, (blk + 1) & 1);
             fetch(kg, blk + 1, kdst, true);
         }
@@ -391,17 +485,19 @@ __global__ __launch_bounds__(256, D == 64 ? (MERGE ? 3 : 4) : 2) void sage_attn_
                 for (int r = 0; r < 16; r++) o[dt][r] *= alpha;
         }
         // V(blk) is in: only K(blk + 1)'s copies were issued after it.
-        if (more)
-            wait_copies<NL + (MERGE ? 1 : 0)>();
-        else
-            wait_copies<0>();
+        if (!shared) {
+            if (more && !ONE)
+                wait_copies<NL + (MERGE ? 1 : 0)>();
+            else
+                wait_copies<0>();
+        }
 #pragma unroll
         for (int d2 = 0; d2 < DT; d2 += 2) {
             uint4 va[2][2];
 #pragma unroll
             for (int e = 0; e < 2; e++) {
-                va[e][0] = *reinterpret_cast<const uint4*>(vt + 16 * 128 * (d2 + e) + voff0);
-                va[e][1] = *reinterpret_cast<const uint4*>(vt + 16 * 128 * (d2 + e) + voff1);
+                va[e][0] = *reinterpret_cast<const uint4*>(vp + 16 * 128 * (d2 + e) + voff0);
+                va[e][1] = *reinterpret_cast<const uint4*>(vp + 16 * 128 * (d2 + e) + voff1);
             }
 #pragma unroll
             for (int e = 0; e < 2; e++) {
@@ -410,94 +506,145 @@ __global__ __launch_bounds__(256, D == 64 ? (MERGE ? 3 : 4) : 2) void sage_attn_
                 o[d2 + e] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, pb, o[d2 + e], 0, 0, 0, 127, 0, 127);
             }
         }
-        wait_reads();
-        if (more) fetch(vg, blk + 1, vdst, false);
+        if (!shared) {
+            wait_reads();
+            if (more) fetch(ONE ? kg : vg, blk + 1, ONE ? kdst : vdst, ONE);
+        }
     };
+    if (HET && whole) {
+        // Every wave has a query group of its own over all blocks, the tiles
+        // shared and double-buffered (two K, two V): the copies of block j + 1
+        // go out behind the barrier that follows block j - 1's last reads.
+        uint8_t* const kb = ldsK;
+        uint8_t* const vb = ONE ? ldsK + 2 * TILE : ldsV;
+        const uint32_t kd = lds_address(kb) + 1024 * wv, vd = lds_address(vb) + 1024 * wv;
+        const uint32_t fkw = 1024 * wv + (D == 128 && (wv & 1) ? fk[1] : fk[0]), fvw = 1024 * wv + fv;
+        auto fetch_shared = [&](int blk) __attribute__((always_inline)) {
+            const uint8_t *tk = kg + (long long)blk * TILE, *tv = vg + (long long)blk * TILE;
+#pragma unroll
+            for (int i = 0; i < TILE / 4096; i++) copy_1k(tk + 4096 * i, fkw, kd + (blk & 1) * TILE + 4096 * i);
+#pragma unroll
+            for (int i = 0; i < TILE / 4096; i++) copy_1k(tv + 4096 * i, fvw, vd + (blk & 1) * TILE + 4096 * i);
+        };
+        fetch_shared(0);
+        for (int blk = 0; blk < nblk; blk++) {
+            wait_copies<0>();
+            block_barrier();
+            if (blk + 1 < nblk) fetch_shared(blk + 1);
+            step(blk, false, true, kb + (blk & 1) * TILE, vb + (blk & 1) * TILE);
+        }
+        const int lw = lane_now(), qw = q0 + (lw & 31);
+        const float inv = 1.0f / sum_halves(l);
+        if (qw >= g.tokens) return;
+        const float* vmean = stats + bhk * 4 * D + D;
+        const float* vscale = vmean + D;
+        uint16_t* orow = out + b * g.o_sb + (long long)qw * g.o_st + h * g.o_sh;
+#pragma unroll
+        for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int d0 = 32 * dt + 8 * j + 4 * (lw >> 5);
+                float y[4];
+#pragma unroll
+                for (int r = 0; r < 4; r++) y[r] = fmaf(o[dt][4 * j + r] * inv, vscale[d0 + r], vmean[d0 + r]);
+                store4(orow + d0, y, g.flags & F_OUT_F16);
+            }
+        return;
+    }
     if (lo < hi) {
-        for (int blk = lo; blk + 1 < hi; blk++) step(blk, true);
-        step(hi - 1, false);
+        for (int blk = lo; blk + 1 < hi; blk++) step(blk, true, false, kt, vt);
+        step(hi - 1, false, false, kt, vt);
     }
 
     wait_copies<0>();  // a wave without blocks has its unused tiles in flight
     // (Lane-derived values are rebuilt here rather than kept over the loop.)
     const int ln = lane_now(), qe = q0 + (ln & 31);
-    // The shares of O, through the waves' own buffers (2 DT groups of four
-    // channels in each, a lane's 16 bytes a group): share p's wave then adds
-    // groups p * GW .. p * GW + GW - 1 of all shares, in key order.
-    constexpr int GW = 4 * DT / S;
-#pragma unroll
-    for (int i = 0; i < 4 * DT; i++) {
-        const int dt = i >> 2, j = i & 3;
-        *reinterpret_cast<float4*>((i < 2 * DT ? kt : vt) + (i % (2 * DT)) * 1024 + ln * 16) =
-            make_float4(o[dt][4 * j], o[dt][4 * j + 1], o[dt][4 * j + 2], o[dt][4 * j + 3]);
-    }
+    // The shares of O, through the waves' own buffers (a group is four channels,
+    // a lane's 16 bytes; 2 DT groups fill a buffer, so one buffer takes two
+    // rounds): every wave writes its shares of a round's groups, then adds all
+    // shares, in key order, of GR / S of them.
+    constexpr int ROUNDS = ONE ? 2 : 1, GR = 4 * DT / ROUNDS;
     ldsE[wv * 64 + ln] = m;
     ldsL[wv * 64 + ln] = sum_halves(l);
-    __syncthreads();
-    if (qe >= g.tokens) return;
-    // m of the last share is the maximum over all keys; a wave without blocks
-    // has its start (or -1e30) and zero shares.
-    const float mend = ldsE[(grp * S + S - 1) * 64 + ln];
-    float f[S], lt = 0.f;
-#pragma unroll
-    for (int i = 0; i < S; i++) {
-        f[i] = __builtin_amdgcn_exp2f(ldsE[(grp * S + i) * 64 + ln] - mend);
-        lt = fmaf(ldsL[(grp * S + i) * 64 + ln], f[i], lt);
-    }
-    const float inv = 1.0f / lt;
+    float f[S], inv = 0.f;
     const float* vmean = stats + bhk * 4 * D + D;
     const float* vscale = vmean + D;
     uint16_t* orow = out + b * g.o_sb + (long long)qe * g.o_st + h * g.o_sh;
 #pragma unroll
-    for (int e = 0; e < GW; e++) {
-        const int i0 = part * GW + e, d0 = 8 * i0 + 4 * (ln >> 5);
-        const uint8_t* src = (i0 < 2 * DT ? ldsK : ldsV) + grp * S * TILE + (i0 % (2 * DT)) * 1024 + ln * 16;
-        float a[4] = {0.f, 0.f, 0.f, 0.f};
+    for (int r = 0; r < ROUNDS; r++) {
+        if (r) __syncthreads();  // the last round's shares are read
 #pragma unroll
-        for (int i = 0; i < S; i++) {
-            const float4 s = *reinterpret_cast<const float4*>(src + i * TILE);
-            a[0] = fmaf(s.x, f[i], a[0]);
-            a[1] = fmaf(s.y, f[i], a[1]);
-            a[2] = fmaf(s.z, f[i], a[2]);
-            a[3] = fmaf(s.w, f[i], a[3]);
+        for (int i = 0; i < GR; i++) {
+            const int gi = r * GR + i, dt = gi >> 2, j = gi & 3;
+            *reinterpret_cast<float4*>((i < 2 * DT ? kt : vt) + (i % (2 * DT)) * 1024 + ln * 16) =
+                make_float4(o[dt][4 * j], o[dt][4 * j + 1], o[dt][4 * j + 2], o[dt][4 * j + 3]);
         }
-        float y[4];
+        __syncthreads();
+        if (r == 0) {
+            // m of the last share is the maximum over all keys; a wave without
+            // blocks has its start (or -1e30) and zero shares.
+            const float mend = ldsE[(grp * S + S - 1) * 64 + ln];
+            float lt = 0.f;
 #pragma unroll
-        for (int c = 0; c < 4; c++) y[c] = fmaf(a[c] * inv, vscale[d0 + c], vmean[d0 + c]);
-        uint2 w;
-        if (g.flags & F_OUT_F16) {
-            w.x = pack_f16x2(y[0], y[1]);
-            w.y = pack_f16x2(y[2], y[3]);
-        } else {
-            w.x = pack_bf16x2(y[0], y[1]);
-            w.y = pack_bf16x2(y[2], y[3]);
+            for (int i = 0; i < S; i++) {
+                f[i] = __builtin_amdgcn_exp2f(ldsE[(grp * S + i) * 64 + ln] - mend);
+                lt = fmaf(ldsL[(grp * S + i) * 64 + ln], f[i], lt);
+            }
+            inv = 1.0f / lt;
         }
-        *reinterpret_cast<uint2*>(orow + d0) = w;
+#pragma unroll
+        for (int e = 0; e < GR / S; e++) {
+            const int i0 = part * (GR / S) + e, d0 = 8 * (r * GR + i0) + 4 * (ln >> 5);
+            const uint8_t* src = (i0 < 2 * DT ? ldsK : ldsV) + grp * S * TILE + (i0 % (2 * DT)) * 1024 + ln * 16;
+            float a[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < S; i++) {
+                const float4 s = *reinterpret_cast<const float4*>(src + i * TILE);
+                a[0] = fmaf(s.x, f[i], a[0]);
+                a[1] = fmaf(s.y, f[i], a[1]);
+                a[2] = fmaf(s.z, f[i], a[2]);
+                a[3] = fmaf(s.w, f[i], a[3]);
+            }
+            if (qe < g.tokens) {
+                float y[4];
+#pragma unroll
+                for (int c = 0; c < 4; c++) y[c] = fmaf(a[c] * inv, vscale[d0 + c], vmean[d0 + c]);
+                store4(orow + d0, y, g.flags & F_OUT_F16);
+            }
+        }
     }
 }
 
 template <int D, bool CAUSAL, bool MERGE, int S>
 static hipError_t launch(const AttendBufs& w, const Geom& g, hipStream_t s) {
     constexpr int ROWS = KEY_WAVES / S * KEY_ROWS;
-    hipLaunchKernelGGL((sage_attn_keys<D, CAUSAL, MERGE, S>), dim3((g.tokens + ROWS - 1) / ROWS, g.heads, g.batch),
+    hipLaunchKernelGGL((sage_attn_keys<D, CAUSAL, MERGE, S, false>), dim3((g.tokens + ROWS - 1) / ROWS, g.heads, g.batch),
                        dim3(64 * KEY_WAVES), 0, s, w.q8, w.q_scale, w.k8, w.k_scale, w.v8, w.stats, w.kbias,
-                       static_cast<uint16_t*>(w.out), g);
+                       static_cast<uint16_t*>(w.out), g, KeyGrid{});
     return hipGetLastError();
 }
-// The combinations key_shares (sage_attention.hip) gives: two shares for
-// merged plans, four for dense ones at head dim 128, either elsewhere.
 template <int D>
-static hipError_t launch_d(int shares, const AttendBufs& w, const Geom& g, hipStream_t s) {
-    if (g.merge > 1) return launch<D, false, true, 2>(w, g, s);
-    if (g.flags & F_CAUSAL)
-        return shares == 4 ? launch<D, true, false, 4>(w, g, s) : launch<D, true, false, 2>(w, g, s);
-    if constexpr (D == 64)
-        if (shares == 2) return launch<D, false, false, 2>(w, g, s);
-    return launch<D, false, false, 4>(w, g, s);
+static hipError_t launch_het(int whole, const AttendBufs& w, const Geom& g, hipStream_t s) {
+    const int n = g.q_tiles * g.heads * g.batch, per = (n + NUM_XCD - 1) / NUM_XCD, w8 = whole / NUM_XCD;
+    hipLaunchKernelGGL((sage_attn_keys<D, false, false, 4, true>), dim3(NUM_XCD * (w8 + 4 * (per - w8))),
+                       dim3(64 * KEY_WAVES), 0, s, w.q8, w.q_scale, w.k8, w.k_scale, w.v8, w.stats, w.kbias,
+                       static_cast<uint16_t*>(w.out), g, KeyGrid{n, w8});
+    return hipGetLastError();
 }
 
-hipError_t launch_attention_keys(int head_dim, int shares, const AttendBufs& w, const Geom& g, hipStream_t s) {
-    return head_dim == 64 ? launch_d<64>(shares, w, g, s) : launch_d<128>(shares, w, g, s);
+// The combinations key_split (sage_attention.hip) gives: two shares for merged
+// and causal plans, four for causal and dense ones, whole tiles beside four
+// shares for dense ones.
+template <int D>
+static hipError_t launch_d(const KeySplit& k, const AttendBufs& w, const Geom& g, hipStream_t s) {
+    if (g.merge > 1) return launch<D, false, true, 2>(w, g, s);
+    if (g.flags & F_CAUSAL)
+        return k.shares == 4 ? launch<D, true, false, 4>(w, g, s) : launch<D, true, false, 2>(w, g, s);
+    return k.whole ? launch_het<D>(k.whole, w, g, s) : launch<D, false, false, 4>(w, g, s);
+}
+
+hipError_t launch_attention_keys(int head_dim, const KeySplit& k, const AttendBufs& w, const Geom& g, hipStream_t s) {
+    return head_dim == 64 ? launch_d<64>(k, w, g, s) : launch_d<128>(k, w, g, s);
 }
 
 }  // namespace sage

@@ -65,9 +65,12 @@ hipError_t launch_attention(int head_dim, const AttendBufs& w, const Geom& g, hi
 // The merged kernels' launch, from the second compilation of the attention
 // source (launch_attention calls it for merged plans).
 hipError_t launch_attention_merged(int head_dim, const AttendBufs& w, const Geom& g, hipStream_t s);
-// The keys-split kernels' launch, two or four shares of the keys a query
-// group (launch_attention calls it for grids of few query tiles).
-hipError_t launch_attention_keys(int head_dim, int shares, const AttendBufs& w, const Geom& g, hipStream_t s);
+// How launch_attention splits the keys (key_split): the shares a query group's
+// keys are split into (0: none), and the 128-query tiles left whole beside them.
+struct KeySplit {
+    int shares, whole;
+};
+hipError_t launch_attention_keys(int head_dim, const KeySplit& k, const AttendBufs& w, const Geom& g, hipStream_t s);
 
 // Whether a forward call on this geometry leaves Q's codes to the attention
 // kernel (F_Q_LATER).

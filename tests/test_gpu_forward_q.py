@@ -16,8 +16,8 @@ pytestmark = pytest.mark.gpu
 # batch, heads, tokens, head_dim, extra Problem arguments, layout: grids of
 # more tiles than the keys-split kernels take.
 CASES = [
-    (1, 54, 1000, 64, {}, "bthd"),
-    (1, 420, 17, 64, dict(dtype=1), "bhtd"),
+    (1, 58, 1000, 64, {}, "bthd"),
+    (1, 450, 17, 64, dict(dtype=1), "bhtd"),
     (2, 11, 1025, 128, dict(dtype=1), "packed"),
     (1, 164, 1, 128, {}, "bthd"),
     (1, 72, 1001, 64, dict(kv_heads=9, causal=True), "bhtd"),
@@ -74,7 +74,7 @@ def test_output_over_q(oracle, torch_gpu, d, where):
     """out = Q in place, and out one head away from Q in one buffer (its rows
     are other heads' queries, still to be read): the same result as apart."""
     torch = torch_gpu
-    h = 420 if d == 64 else 164
+    h = 475 if d == 64 else 240
     S, p, sa, ws, ts, opts = _setup(torch, oracle, 1, h, 130, d, {}, "bthd")
     o = torch.empty_like(ts[0])
     sa.prepare(ws, *(S.Tensor(t) for t in ts), opts)
@@ -92,11 +92,11 @@ def test_refused_output_leaves_a_prepared_workspace(oracle, torch_gpu):
     """An output that attend refuses: forward reports attend's text, and the
     workspace holds prepare's codes, as after the two calls."""
     torch = torch_gpu
-    S, p, sa, ws, ts, opts = _setup(torch, oracle, 1, 54, 1000, 64, {}, "bthd")
+    S, p, sa, ws, ts, opts = _setup(torch, oracle, 1, 58, 1000, 64, {}, "bthd")
     tens = [S.Tensor(t) for t in ts]
     short = torch.empty(64, dtype=ts[0].dtype, device="cuda")
     with pytest.raises(S.SageError, match="output holds 64 elements"):
-        sa.forward(ws, *tens, S.TensorMut(short, S.Strides.bthd(1000, 54, 64)), opts)
+        sa.forward(ws, *tens, S.TensorMut(short, S.Strides.bthd(1000, 58, 64)), opts)
     o1, o2 = torch.empty_like(ts[0]), torch.empty_like(ts[0])
     sa.attend(ws, S.TensorMut(o1))
     sa.forward(ws, *tens, S.TensorMut(o2), opts)
@@ -111,7 +111,7 @@ def test_special_queries(oracle, torch_gpu, d, dtype):
     subnormals (127 / amax overflows in bf16), the largest finite value, and
     ties of the rounding: the codes and scales equal the prologue's."""
     torch = torch_gpu
-    h = 420 if d == 64 else 164
+    h = 475 if d == 64 else 240
     S, p, sa, ws, ts, opts = _setup(torch, oracle, 1, h, 200, d, dict(dtype=dtype), "bthd")
     q = ts[0].view(torch.int16)
     bits = lambda x: int(np.uint16(x).view(np.int16))  # noqa: E731

@@ -1,7 +1,8 @@
 """The attention kernels on both sides of the line between split and whole keys.
 
 Grids of few query tiles run the kernel that splits a query group's keys over
-two or four waves; larger ones the whole-key kernels. Each case sits at a place
+two or four waves; larger ones the whole-key kernels, with a remainder of tiles
+over a whole number a CU split beside whole ones. Each case sits at a place
 where the split can go wrong: fewer key blocks than shares, a ragged last
 block, blocks past the 64 whose scales a wave holds at a time, causal groups
 whose last share is the diagonal alone, grouped heads, merged biases, and a
@@ -27,7 +28,11 @@ SPLIT = [
     (2, 5, 257, 64, dict(kv_heads=1, dtype=1)),
     (1, 1, 4500, 64, {}),                                # 71 blocks: two chunks of K scales
     (1, 1, 8200, 128, dict(dtype=1)),                    # 129 blocks, the last one of 8 keys
-    (1, 40, 1000, 64, {}),                               # two shares (320 tiles)
+    (1, 34, 1000, 64, {}),                               # 256 tiles whole, 16 split
+    (1, 5, 7000, 64, dict(dtype=1)),                     # 275 tiles: uneven XCD ranges
+    (2, 33, 1003, 64, dict(kv_heads=11)),                # 512 whole, 16 split
+    (1, 5, 6700, 128, {}),                               # 265: one buffer a wave
+    (3, 30, 700, 128, dict(dtype=1)),                    # 512 whole, 28 split
     (1, 2, 4170, 128, dict(causal=True)),
     (3, 4, 700, 64, dict(kv_heads=2, causal=True)),
     (1, 8, 1000, 64, dict(causal=True)),                 # dealt longest first
@@ -37,7 +42,7 @@ SPLIT = [
     (2, 2, 50 * 95, 128, dict(merge=4, layout=(50, 5, 9, 10, 0))),
 ]
 WHOLE = [
-    (1, 54, 1000, 64, {}),
+    (1, 58, 1000, 64, {}),
     (1, 21, 1000, 128, dict(dtype=1)),
     (1, 72, 1001, 64, dict(kv_heads=9, causal=True)),
     (2, 20, 1050, 128, dict(causal=True)),
