@@ -93,4 +93,37 @@ __device__ __forceinline__ int lane_now() {
     return (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
 }
 
+__device__ __forceinline__ uint32_t lds_address(const void* p) {
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)(uintptr_t)(__attribute__((address_space(3))) const void*)p);
+}
+
+// Brings K and V of keys 32 gi .. 32 gi + 31 of a head (kg, vg: the head's code
+// arrays, `bytes` each) into this XCD's L2: one dword of every 128-byte line,
+// copied to an LDS sink that nobody reads. Each 32-query group of a head calls
+// it once for its own share, so a head's codes are on their way at once instead
+// of a block ahead of the first wave that needs them: with few waves a SIMD a
+// block takes less time than a miss. Four frames (352 tiles) 61.2 -> 58.3 us a
+// forward, one frame 19.3 -> 18.8; sage_attn, whose blocks take longer, lost 2
+// to 3% to it at 384 and 768 tiles. It is older than every copy that the
+// caller counts, so those waits hold; the caller waits for it before it uses
+// the sink's memory. Only for heads of up to WARM_BYTES of K: an XCD's 4 MB L2 holds the K and V of
+// the heads its workgroups are on, and a longer head's would be gone again
+// before the sweep reaches them.
+constexpr long long WARM_BYTES = 3LL << 19;
+template <int D>
+__device__ __forceinline__ void warm_l2(const uint8_t* kg, const uint8_t* vg, long long bytes, int gi, uint32_t sink) {
+    const int ln = lane_now();
+    const long long off = 32LL * D * gi + 128 * (ln % (D / 4));
+    if (ln < D / 2 && off < bytes) {
+        [[maybe_unused]] const uint8_t* p = (ln < D / 4 ? kg : vg) + off;
+#if defined(__HIP_DEVICE_COMPILE__)
+        asm volatile(
+            "s_mov_b32 m0, %0\n\t"
+            "s_nop 0\n\t"
+            "global_load_lds_dword %1, off" ::"s"(__builtin_amdgcn_readfirstlane((int)sink)), "v"(p)
+            : "memory");
+#endif
+    }
+}
+
 }  // namespace sage

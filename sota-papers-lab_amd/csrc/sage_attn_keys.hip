@@ -48,9 +48,6 @@ constexpr int KEY_ROWS = 32;  // queries a group
 // nothing else in the kernel waits for them. (M0, the copies' LDS base, is a
 // register the compiler sets anew before each of its own uses; a kernel that
 // uses these helpers has none.)
-__device__ __forceinline__ uint32_t lds_address(const void* p) {
-    return (uint32_t)__builtin_amdgcn_readfirstlane((int)(uintptr_t)(__attribute__((address_space(3))) const void*)p);
-}
 // 4 KB, four copies of 64 lanes x 16 bytes: copy i reads base + 1024 i + even
 // (odd copies: + odd) and fills dst + 1024 i + 16 lane.
 __device__ __forceinline__ void copy_4k(const uint8_t* base, uint32_t even, uint32_t odd, uint32_t dst) {
@@ -198,6 +195,8 @@ __global__ __launch_bounds__(256, D == 64 ? (MERGE ? 3 : 4) : (HET ? 3 : 2)) voi
     const uint8_t* kg = reinterpret_cast<const uint8_t*>(k8) + bhk * (long long)g.tk_pad * D;
     const uint8_t* vg = v8 + bhk * (long long)g.tk_pad * D;
     const float* ksc = k_scale + bhk * g.kblocks;
+    if ((whole || part == 0) && (long long)g.tk_pad * D <= WARM_BYTES)
+        warm_l2<D>(kg, vg, (long long)g.tk_pad * D, q0 / 32, lds_address(ldsE + wv * 64));  // its own slot
     uint8_t* const kt = ldsK + wv * TILE;
     uint8_t* const vt = ldsV + wv * TILE;
     const uint32_t bdst = MERGE ? lds_address(ldsB + wv * 2 * BN) : 0;
@@ -556,7 +555,7 @@ __global__ __launch_bounds__(256, D == 64 ? (MERGE ? 3 : 4) : (HET ? 3 : 2)) voi
         step(hi - 1, false, false, kt, vt);
     }
 
-    wait_copies<0>();  // a wave without blocks has its unused tiles in flight
+    wait_copies<0>();  // a wave without blocks has its unused tiles (and the warm-up) in flight
     // (Lane-derived values are rebuilt here rather than kept over the loop.)
     const int ln = lane_now(), qe = q0 + (ln & 31);
     // The shares of O, through the waves' own buffers (a group is four channels,
