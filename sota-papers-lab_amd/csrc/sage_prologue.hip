@@ -58,7 +58,7 @@ __device__ __forceinline__ void store16_once(void* p, uint4 w) {
 // LayerNorm of one head row (sage_quant.cu:34-52) whose D channels lie on
 // D/8 consecutive lanes, 8 a lane (ch = lane's chunk); every lane of the wave
 // calls it. The lane sums meet in the reference's xor butterfly over
-// distances 1 .. D/16; the square deviations accumulate fused (fmaf), the
+// distances 1 .. D/16 (row_sum); the square deviations accumulate fused (fmaf), the
 // variance takes fmaf(s2, 1/D, eps) and the output fmaf((x - mean) * rstd,
 // w, b) -- the reference's expressions under NVRTC's default contraction.
 // rstd is 1 / sqrt(.) with the square root and the divide each correctly
@@ -71,8 +71,7 @@ __device__ __forceinline__ void layernorm8(float* x, const float* __restrict__ w
     float s = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; e++) s += x[e];
-#pragma unroll
-    for (int o = 1; o < CH; o <<= 1) s += __shfl_xor(s, o, 64);
+    s = row_sum<CH>(s);
     const float mean = s * (1.0f / D);
     float s2 = 0.f;
 #pragma unroll
@@ -80,8 +79,7 @@ __device__ __forceinline__ void layernorm8(float* x, const float* __restrict__ w
         const float d = x[e] - mean;
         s2 = __builtin_fmaf(d, d, s2);
     }
-#pragma unroll
-    for (int o = 1; o < CH; o <<= 1) s2 += __shfl_xor(s2, o, 64);
+    s2 = row_sum<CH>(s2);
     const float rstd = rsqrt_rn2(__builtin_fmaf(s2, 1.0f / D, eps));
 #pragma unroll
     for (int e = 0; e < 8; e++) x[e] = __builtin_fmaf((x[e] - mean) * rstd, w[ch * 8 + e], bias[ch * 8 + e]);
@@ -368,8 +366,18 @@ __global__ __launch_bounds__(256) void sage_prep(const uint16_t* __restrict__ q,
     __shared__ float ginv[QTILE / QGROUP];
     __shared__ float red[8][4][D];
     constexpr int STATS = stat_roles<QKV>();
-    const int roles = STATS + (g.flags & F_Q_LATER ? 0 : g.group), tile = (int)blockIdx.x / roles, role = (int)blockIdx.x % roles;
-    const int hk = blockIdx.y, b = blockIdx.z;
+    const int roles = STATS + (g.flags & F_Q_LATER ? 0 : g.group);
+    int tile = (int)blockIdx.x / roles, role = (int)blockIdx.x % roles, hk = blockIdx.y, b = blockIdx.z;
+    if constexpr (QKV) {
+        // All K roles first, then Q's, V's light ones last.
+        const unsigned per = (unsigned)g.q_tiles * gridDim.y * gridDim.z;
+        const unsigned lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+        const unsigned ord = lin / per, rest = lin % per;
+        role = ord == 0 ? 0 : ord == (unsigned)roles - 1 ? 1 : (int)ord + 1;
+        tile = (int)(rest % g.q_tiles);
+        hk = (int)(rest / g.q_tiles % gridDim.y);
+        b = (int)(rest / g.q_tiles / gridDim.y);
+    }
     if (role >= STATS) {
         tile_q8<D, LN, QKV>(q, ln, q8, q_scale, g, qa, tile, hk, role - STATS, b, gmax, ginv);
     } else if constexpr (!QKV) {
