@@ -207,7 +207,19 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : (MERGE ? 2 : 3)) void sage_attn(
         // XCD x holds head slots [x * hx, (x + 1) * hx); its i-th workgroup
         // takes query tile ntq - 1 - i / hx of head slot x * hx + i % hx, so
         // the XCD deals its tiles longest first across all of its heads.
-        const int per = total / NUM_XCD, hx = per / ntq, x = lin % NUM_XCD, i = lin / NUM_XCD;
+        const int per = total / NUM_XCD, hx = per / ntq, x = lin % NUM_XCD;
+        int i = lin / NUM_XCD;
+        // Where all workgroups are resident at once, workgroup i and i + 32 of
+        // an XCD share a CU (the dispatcher walks its 32 CUs), and dealt
+        // longest first throughout the first CUs get the longest of every
+        // batch. Reversing every other batch evens the CUs' sums (D 64 768
+        // tiles N 4096 65.0 -> 58.6 us, 1024 N 16384 257 -> 234; D 128 704 N
+        // 1400 40.2 -> 36.9); with more workgroups the later ones go where
+        // one has ended, and the order makes no difference.
+        if (per <= 32 * (D == 64 ? 4 : 3)) {
+            const int b0 = i & ~31;
+            if ((i & 32) == 0) i = b0 + min(32, per - b0) - 1 - (i - b0);
+        }
         qt = ntq - 1 - i / hx;
         hb = x * hx + i % hx;
     } else {
@@ -932,10 +944,11 @@ static hipError_t resources_of(int head_dim, int* regs, int* spill, int* lds) {
 //   D 64        96 tiles N 689: 11.8 / 8.0 / 9.1     176, N 1378: 19.9 / 16.7 / 19.0
 //               216, N 1100: 18.2 / 17.9             256, N 1000: 17.3 / 17.2 / 17.1
 //   D 64 causal 256, N 1000: 16.3 / 11.5 / 12.9      352, N 2756: 36.2 / 27.6 / 28.6
-//               480, N 5000: 81.3 / 67.8 / 63.2      704, N 5512: 78.5 / 84.5 / 79.8
+//               480, N 5000: 81.3 / 67.8 / 63.2      512, N 1000: 18.4 / 22.1 / 18.9
 //   D 128       128, N 8192: 118 / 76.9 / 84.7       176, N 1378: 27.6 / 27.5 / 27.8
 //   D 128 causal 176, N 1378: 26.8 / 20.7 / 21.2     256, N 1000: 22.3 / 21.5 / 18.9
 //               352, N 2756: 49.3 / 47.7 / 43.9      384, N 689: 18.0 / 24.5 / 21.8
+//               320, N 1000: 23.2 / - / 25.4         (whole tiles in sage_attn's paired order)
 //   merged      D 64 96 tiles, stride 2: 7.2 / 6.2 / 6.4, stride 4: 5.5 / 5.7 / 5.3;
 //               D 128 96, stride 2: 9.8 / 8.6 / 8.7, stride 4: 8.2 / 8.2 / 7.1;
 //               352 D 64: 21.9 / 23.4 / 21.9, D 128: 29.8 / 41.5 / 37.9
@@ -960,8 +973,8 @@ static KeySplit key_split(int head_dim, const Geom& g) {
     const long long n = (long long)g.q_tiles * g.heads * g.batch;
     if (g.merge > 1) return {n <= (head_dim == 64 ? 224 : 128) ? 2 : 0, 0};
     if (g.flags & F_CAUSAL) {
-        if (head_dim == 64) return {n <= 320 ? 4 : n <= 560 ? 2 : 0, 0};
-        return {n <= 208 ? 4 : n <= 320 ? 2 : 0, 0};
+        if (head_dim == 64) return {n <= 320 ? 4 : n <= 480 ? 2 : 0, 0};
+        return {n <= 208 ? 4 : n <= 288 ? 2 : 0, 0};
     }
     if (n <= (head_dim == 64 ? 224 : 160)) return {4, 0};
     // The largest remainder that is split beside 1, 2, .. tiles a CU.
