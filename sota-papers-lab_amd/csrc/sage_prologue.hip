@@ -31,6 +31,7 @@
 // the q8, k8 and v8 stores. The attention kernel shares its K/V tiles through
 // L2, not through that cache.
 #include <algorithm>
+#include <type_traits>
 
 #include "sage_device.hpp"
 #include "sage_internal.hpp"
@@ -569,13 +570,22 @@ __device__ __forceinline__ void put_v(uint8_t* vt, int ch, int kl, const float* 
 // `sum * rc - mean`, equal to the dense (k + 0) - mean when n = 1.
 // Under QK LayerNorm (LN) each K row (each member, when merging) is
 // normalised before it is summed (sage_quant.cu:271).
-template <int D, bool LN, bool QKV>
-__global__ __launch_bounds__(256) void sage_quant_kv(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v,
-                                                     const float* __restrict__ ln,
-                                                     float* __restrict__ stats, int8_t* __restrict__ k8,
-                                                     float* __restrict__ k_scale, uint8_t* __restrict__ v8,
-                                                     float* __restrict__ kbias, const float* __restrict__ part,
-                                                     Geom g, QkvDev qa) {
+//
+// Merged plans have instantiations of their own: the member gathers' registers
+// took waves from every plain plan (normed rows, D = 64: 105 registers -> 80,
+// 8 x 689 tokens of 16 heads 14.8 -> 12.3 us; fused rows 140 -> 69; plain
+// D = 128, 2 x 32 heads x 4096 tokens 35.8 -> 35.2 us). EARLY, for plain
+// D = 128 rows of plans short enough to fold the statistics here, loads the
+// rows before the fold (2 x 1000 tokens of 32 heads: 0.3 us of the call's
+// 41.2); without a fold that cost 2 us in 36 at 4096 tokens, and at D = 64 0.4
+// in 12. Four waves a SIMD is asked for where the registers land just above
+// that line.
+template <int D, bool LN, bool QKV, bool MERGE, bool EARLY>
+__global__ __launch_bounds__(256, MERGE && (LN || D == 128) ? 1 : 4)
+void sage_quant_kv(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const float* __restrict__ ln,
+                   float* __restrict__ stats, int8_t* __restrict__ k8, float* __restrict__ k_scale,
+                   uint8_t* __restrict__ v8, float* __restrict__ kbias, const float* __restrict__ part, Geom g,
+                   QkvDev qa) {
     constexpr int CH = D / 8;
     constexpr int TPI = 256 / CH;
     constexpr int NI = KBLOCK / TPI;
@@ -589,9 +599,22 @@ __global__ __launch_bounds__(256) void sage_quant_kv(const uint16_t* __restrict_
     __shared__ float fold[4 * D];
     if (tid == 0) kmax = 0u;
 
+    constexpr int RAW = QKV || MERGE ? 1 : NI;
+    uint4 kraw[RAW], vraw[RAW];
+    auto load_rows = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < RAW; i++) {
+            const int j = blk * KBLOCK + slot + i * TPI;
+            const bool ok = j < g.tk;
+            kraw[i] = load16(k + b * g.k_sb + (long long)j * g.k_st + hk * g.k_sh + ch * 8, ok);
+            vraw[i] = load16(v + b * g.v_sb + (long long)j * g.v_st + hk * g.v_sh + ch * 8, ok);
+        }
+    };
+    if constexpr (EARLY) load_rows();
+
     const float* st = stats + bhk * 4 * D;
     float mk[8], mv[8], iv[8];
-    if (part) {
+    if (EARLY || part) {
         fold_tiles<D>(part + bhk * g.q_tiles * 4 * D, stats + bhk * 4 * D, g, blk == 0, fold);
 #pragma unroll
         for (int e = 0; e < 8; e++) {
@@ -621,7 +644,7 @@ __global__ __launch_bounds__(256) void sage_quant_kv(const uint16_t* __restrict_
     // A block with no key past the sequence (all but a ragged last one) can
     // run without the per-key guards (workgroup-uniform).
     const bool full = (blk + 1) * KBLOCK <= g.tk;
-    if (QKV && g.merge == 1) {
+    if constexpr (QKV && !MERGE) {
         // Rows of the fused projection: V first, then K, so that only one
         // part's channel constants (QkvLane) and statistics are live at a time.
         __syncthreads();
@@ -651,11 +674,11 @@ __global__ __launch_bounds__(256) void sage_quant_kv(const uint16_t* __restrict_
         // K rows as sage_prep stashed them (bf16, after the QKV arithmetic),
         // over this block's k8 and v8 bytes: every read here is consumed
         // before the K-scale barrier, every code store comes after it.
-        uint4 kraw[NI];
+        uint4 kst[NI];
 #pragma unroll
         for (int i = 0; i < NI; i++) {
             const int j = blk * KBLOCK + slot + i * TPI;
-            kraw[i] = j < g.tk ? *reinterpret_cast<const uint4*>(k_stash(k8, v8, g, bhk, j, ch, D))
+            kst[i] = j < g.tk ? *reinterpret_cast<const uint4*>(k_stash(k8, v8, g, bhk, j, ch, D))
                                : make_uint4(0, 0, 0, 0);
         }
 #pragma unroll
@@ -663,7 +686,7 @@ __global__ __launch_bounds__(256) void sage_quant_kv(const uint16_t* __restrict_
             const int kl = slot + i * TPI;
             const bool ok = blk * KBLOCK + kl < g.tk;
             float fk[8];
-            unpack8(kraw[i], fk, false);
+            unpack8(kst[i], fk, false);
             if (LN) layernorm8<D>(fk, ln + 2 * D, ln + 3 * D, ch, g.ln_eps);
 #pragma unroll
             for (int e = 0; e < 8; e++) {
@@ -671,15 +694,8 @@ __global__ __launch_bounds__(256) void sage_quant_kv(const uint16_t* __restrict_
                 amax = fmaxf(amax, fabsf(kv[i][e]));
             }
         }
-    } else if (g.merge == 1) {
-        uint4 kraw[NI], vraw[NI];
-#pragma unroll
-        for (int i = 0; i < NI; i++) {
-            const int j = blk * KBLOCK + slot + i * TPI;
-            const bool ok = j < g.tk;
-            kraw[i] = load16(k + b * g.k_sb + (long long)j * g.k_st + hk * g.k_sh + ch * 8, ok);
-            vraw[i] = load16(v + b * g.v_sb + (long long)j * g.v_st + hk * g.v_sh + ch * 8, ok);
-        }
+    } else if constexpr (!MERGE) {
+        if (!EARLY) load_rows();
         __syncthreads();
         auto rows = [&](bool all) __attribute__((always_inline)) {
 #pragma unroll
@@ -787,20 +803,41 @@ __global__ __launch_bounds__(256) void sage_quant_kv(const uint16_t* __restrict_
             float ks[8], vs[8];
 #pragma unroll
             for (int e = 0; e < 8; e++) ks[e] = vs[e] = 0.f;
-            for (int m = 0; m < cells; m++) {
-                const bool mok = m < cnt;
-                const int tok = base + (mok ? (m / nx) * g.grid_w + m % nx : 0);
-                float fk[8], fv[8];
-                unpack8(load16(k + b * g.k_sb + (long long)tok * g.k_st + hk * g.k_sh + ch * 8, mok), fk, f16);
-                unpack8(load16(v + b * g.v_sb + (long long)tok * g.v_st + hk * g.v_sh + ch * 8, mok), fv, f16);
-                if (LN) layernorm8<D>(fk, ln + 2 * D, ln + 3 * D, ch, g.ln_eps);
-                if (mok) {
+            // Member y nx + x is token base + y grid_w + x, and the members are
+            // summed in that order. A row of the cell at a time (merge is 2 or
+            // 4), its loads issued together, and only the rows the key has:
+            // one member at a time each wave waited out up to sixteen load
+            // latencies a key, dense keys' included (40 frames of 880 tokens,
+            // 16 heads, merge 4: 35.6 -> 27.1 us, 4.2 TB/s; two rows at a time
+            // 46.9, their registers leave two waves a SIMD). The norm's sums
+            // are over the D/8 lanes of one key, which run the same rows.
+            const uint16_t* kp = k + b * g.k_sb + (long long)base * g.k_st + hk * g.k_sh + ch * 8;
+            const uint16_t* vp = v + b * g.v_sb + (long long)base * g.v_st + hk * g.v_sh + ch * 8;
+            for (int y = 0; y * nx < cnt; y++) {
+                uint4 kr[4], vr[4];
 #pragma unroll
-                    for (int e = 0; e < 8; e++) {
-                        ks[e] += fk[e];
-                        vs[e] += fv[e];
+                for (int x = 0; x < 4; x++)
+                    if (x < g.merge) {
+                        const long long off = (long long)y * g.grid_w + x;
+                        const bool mok = x < nx && y * nx + x < cnt;
+                        kr[x] = load16(kp + off * g.k_st, mok);
+                        vr[x] = load16(vp + off * g.v_st, mok);
                     }
-                }
+#pragma unroll
+                for (int x = 0; x < 4; x++)
+                    if (x < g.merge) {
+                        float fk[8], fv[8];
+                        unpack8(kr[x], fk, f16);
+                        unpack8(vr[x], fv, f16);
+                        if (LN) layernorm8<D>(fk, ln + 2 * D, ln + 3 * D, ch, g.ln_eps);
+                        if (x < nx && y * nx + x < cnt) {
+#pragma unroll
+                            for (int e = 0; e < 8; e++) {
+                                ks[e] += fk[e];
+                                vs[e] += fv[e];
+                            }
+                        }
+                    }
             }
             const float rc = cnt > 0 ? 1.0f / (float)cnt : 0.f;
             float vq[8];
@@ -927,8 +964,22 @@ static hipError_t launch_prologue_d(const uint16_t* q, const uint16_t* k, const 
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    hipLaunchKernelGGL((sage_quant_kv<D, LN, QKV>), dim3(g.kblocks, g.kv_heads, g.batch), dim3(256), 0, s, k, v, ln,
-                       w.stats, w.k8, w.k_scale, w.v8, w.kbias, fold ? w.part : nullptr, g, qa);
+    auto quant = [&](auto merge, auto early) {
+        hipLaunchKernelGGL((sage_quant_kv<D, LN, QKV, decltype(merge)::value, decltype(early)::value>),
+                           dim3(g.kblocks, g.kv_heads, g.batch), dim3(256), 0, s, k, v, ln, w.stats, w.k8, w.k_scale,
+                           w.v8, w.kbias, fold ? w.part : nullptr, g, qa);
+    };
+    if (g.merge > 1) {
+        quant(std::true_type{}, std::false_type{});
+        return hipGetLastError();
+    }
+    if constexpr (D == 128 && !QKV) {
+        if (fold) {
+            quant(std::false_type{}, std::true_type{});
+            return hipGetLastError();
+        }
+    }
+    quant(std::false_type{}, std::false_type{});
     return hipGetLastError();
 }
 

@@ -110,3 +110,18 @@ def test_merged_attention_equals_dense_on_uniform_cells(oracle, torch_gpu, strid
     for out in (merged_out, dense_out):
         e64 = oracle.errors(out, exact)
         assert e64["cos"] > 0.999 and e64["rel_l2"] < 0.04, e64
+
+
+# Cells cut by the grid's edge in either direction (1 to 3 columns or rows
+# left of a cell of 4, 1 of a cell of 2), grids narrower than a cell, special
+# tokens between merged frames, and normed rows beside plain ones.
+@pytest.mark.parametrize("grid", [(4, 4), (5, 6), (7, 3), (2, 9), (1, 1), (3, 21)])
+@pytest.mark.parametrize("stride,d,norm", [(2, 64, False), (4, 64, True), (2, 128, True), (4, 128, False)])
+def test_merged_codes_over_cut_cells(oracle, torch_gpu, grid, stride, d, norm):
+    from test_oracle_qknorm import ln_params
+
+    kw = {"ln": ln_params(oracle, d, 3)} if norm else {"dtype": 1}
+    p = _merged(oracle, stride, (4, 3, *grid, 1), 4, d, kv_heads=2, **kw)
+    q, k, v = oracle.generate(p, oracle.GenSpec(k_off_std=2.0, seed=sum(grid)))
+    pro, _ = run(torch_gpu, p, q, k, v)
+    assert_prologue_equal(pro, oracle.prologue(p, q, k, v))
