@@ -292,20 +292,37 @@ def v8_position(k: int) -> int:
 # ------------------------------------------------------------------ tensors
 
 
-def _dtype_code(t) -> int:
-    import torch
+_codes = None
 
-    if t.dtype == torch.bfloat16:
-        return BF16
-    if t.dtype == torch.float16:
-        return F16
-    raise SageError(1, f"sage tensors are bf16 or fp16, got {t.dtype}")
+
+def _dtype_code(t) -> int:
+    global _codes
+    if _codes is None:
+        import torch
+
+        _codes = {torch.bfloat16: BF16, torch.float16: F16}
+    code = _codes.get(t.dtype)
+    if code is None:
+        raise SageError(1, f"sage tensors are bf16 or fp16, got {t.dtype}")
+    return code
 
 
 def _elems_from(t) -> int:
     """Elements from the view's first element to the end of its storage."""
-    es = t.element_size()
-    return t.untyped_storage().nbytes() // es - t.storage_offset()
+    return t.untyped_storage().nbytes() // t.element_size() - t.storage_offset()
+
+
+# A forward makes four of these, and the smallest calls are as long on the host
+# as on the GPU: one stride() call and the nested struct from a tuple take
+# 0.9 us a tensor where a Strides, its struct and three stride(i) took 1.45
+# (2 heads of 256 tokens: a forward 17.4 -> 15.4 us).
+def _tensor_c(cls, t, strides):
+    if strides is None:
+        st = t.stride()
+        st = (st[0], st[1], st[2])
+    else:
+        st = (strides.batch, strides.token, strides.head)
+    return cls(t.data_ptr(), _elems_from(t), st, _dtype_code(t))
 
 
 @dataclass
@@ -316,9 +333,7 @@ class Tensor:
     strides: Optional[Strides] = None
 
     def _c(self) -> _abi.sage_tensor:
-        t = self.data
-        st = self.strides or Strides(t.stride(0), t.stride(1), t.stride(2))
-        return _abi.sage_tensor(t.data_ptr(), _elems_from(t), st._c(), _dtype_code(t))
+        return _tensor_c(_abi.sage_tensor, self.data, self.strides)
 
 
 @dataclass
@@ -329,9 +344,7 @@ class TensorMut:
     strides: Optional[Strides] = None
 
     def _c(self) -> _abi.sage_tensor_mut:
-        t = self.data
-        st = self.strides or Strides(t.stride(0), t.stride(1), t.stride(2))
-        return _abi.sage_tensor_mut(t.data_ptr(), _elems_from(t), st._c(), _dtype_code(t))
+        return _tensor_c(_abi.sage_tensor_mut, self.data, self.strides)
 
 
 # ------------------------------------------------------------------ engine
