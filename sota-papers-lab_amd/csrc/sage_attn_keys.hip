@@ -45,42 +45,58 @@ constexpr int KEY_ROWS = 32;  // queries a group
 // its count (they complete in order). The compiler tracks its own copies
 // object by object but loses that over a loop (it waited for V's copies before
 // every read of K), so the copies are written out, with every wait explicit:
-// nothing else in the kernel waits for them. (M0, the copies' LDS base, is a
-// register the compiler sets anew before each of its own uses; a kernel that
-// uses these helpers has none.)
+// nothing else in the kernel waits for them.
+// The base goes through an SGPR pair that a scalar move writes inside the
+// statement: a vector memory instruction may read an SGPR only five wait states
+// after a vector instruction wrote it, the compiler keeps no such distance to
+// an asm statement, and a base restored from a vector register's lanes
+// (v_readlane) arrives right before it. A scalar read of that SGPR is
+// interlocked, and a scalar write needs no wait before the load. (s_nop: one
+// wait state between M0's write, the copies' LDS base, and the load.)
 // 4 KB, four copies of 64 lanes x 16 bytes: copy i reads base + 1024 i + even
 // (odd copies: + odd) and fills dst + 1024 i + 16 lane.
 __device__ __forceinline__ void copy_4k(const uint8_t* base, uint32_t even, uint32_t odd, uint32_t dst) {
 #if defined(__HIP_DEVICE_COMPILE__)
+    const uint8_t* b;
     asm volatile(
-        "s_mov_b32 m0, %0\n\t"
+        "s_mov_b64 %0, %4\n\t"
+        "s_mov_b32 m0, %1\n\t"
         "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %1, %3\n\t"
-        "global_load_lds_dwordx4 %2, %3 offset:1024\n\t"
-        "global_load_lds_dwordx4 %1, %3 offset:2048\n\t"
-        "global_load_lds_dwordx4 %2, %3 offset:3072" ::"s"(__builtin_amdgcn_readfirstlane((int)dst)),
-        "v"(even), "v"(odd), "s"(base)
-        : "memory");
+        "global_load_lds_dwordx4 %2, %0\n\t"
+        "global_load_lds_dwordx4 %3, %0 offset:1024\n\t"
+        "global_load_lds_dwordx4 %2, %0 offset:2048\n\t"
+        "global_load_lds_dwordx4 %3, %0 offset:3072"
+        : "=&s"(b)
+        : "s"(__builtin_amdgcn_readfirstlane((int)dst)), "v"(even), "v"(odd), "s"(base)
+        : "memory", "m0");
 #endif
 }
 // 1 KB, 16 bytes a lane.
 __device__ __forceinline__ void copy_1k(const uint8_t* base, uint32_t off, uint32_t dst) {
 #if defined(__HIP_DEVICE_COMPILE__)
+    const uint8_t* b;
     asm volatile(
-        "s_mov_b32 m0, %0\n\t"
+        "s_mov_b64 %0, %3\n\t"
+        "s_mov_b32 m0, %1\n\t"
         "s_nop 0\n\t"
-        "global_load_lds_dwordx4 %1, %2" ::"s"(__builtin_amdgcn_readfirstlane((int)dst)), "v"(off), "s"(base)
-        : "memory");
+        "global_load_lds_dwordx4 %2, %0"
+        : "=&s"(b)
+        : "s"(__builtin_amdgcn_readfirstlane((int)dst)), "v"(off), "s"(base)
+        : "memory", "m0");
 #endif
 }
 // 256 bytes, four a lane.
 __device__ __forceinline__ void copy_256(const uint8_t* base, uint32_t off, uint32_t dst) {
 #if defined(__HIP_DEVICE_COMPILE__)
+    const uint8_t* b;
     asm volatile(
-        "s_mov_b32 m0, %0\n\t"
+        "s_mov_b64 %0, %3\n\t"
+        "s_mov_b32 m0, %1\n\t"
         "s_nop 0\n\t"
-        "global_load_lds_dword %1, %2" ::"s"(__builtin_amdgcn_readfirstlane((int)dst)), "v"(off), "s"(base)
-        : "memory");
+        "global_load_lds_dword %2, %0"
+        : "=&s"(b)
+        : "s"(__builtin_amdgcn_readfirstlane((int)dst)), "v"(off), "s"(base)
+        : "memory", "m0");
 #endif
 }
 // At most N of the wave's vector memory operations are outstanding.

@@ -1,0 +1,96 @@
+"""The machine code of the kernels that carry inline assembly, on the CPU.
+
+The compiler puts no wait states around an instruction inside an asm statement.
+On gfx9 a vector memory instruction may read an SGPR that a vector instruction
+(v_readlane, v_readfirstlane, a compare) wrote only five wait states later;
+sooner it can see the old value, i.e. an address of two halves that do not
+belong together. A base pointer reaches such an asm straight from v_readlane
+whenever the register allocator parks SGPRs in lanes of a vector register, so
+the source alone does not show it: this test compiles the unit as the build
+does and reads the assembly."""
+from __future__ import annotations
+
+import re
+import subprocess
+
+import pytest
+
+import build as hip_build  # sota-papers-lab_amd/build.py
+
+WAIT_STATES = 5  # VALU writes an SGPR, a VMEM instruction reads it
+
+
+def _sgprs(text: str) -> set:
+    out = {int(x) for x in re.findall(r"\bs(\d+)\b", text)}
+    for a, b in re.findall(r"\bs\[(\d+):(\d+)\]", text):
+        out |= set(range(int(a), int(b) + 1))
+    if "vcc" in text:
+        out |= {"vcc"}
+    return out
+
+
+def sgpr_hazards(asm: str, need: int = WAIT_STATES) -> list:
+    """(line, text) of every VMEM instruction that reads an SGPR fewer than
+    `need` wait states after a VALU instruction wrote it, along straight-line
+    code (a taken branch costs more than five)."""
+    age, found = {}, []  # SGPR -> wait states since a VALU wrote it
+    for n, line in enumerate(asm.splitlines(), 1):
+        t = line.split(";")[0].strip()
+        if not t or t.startswith(".") or t.startswith("//"):
+            continue
+        if t.endswith(":"):
+            if not t.startswith(".L"):
+                age = {}  # another function
+            continue
+        op, _, args = t.partition(" ")
+        if re.match(r"(global|buffer|flat|scratch)_", op):
+            if any(age.get(r, need) < need for r in _sgprs(args)):
+                found.append((n, t))
+        step = int(args, 0) + 1 if op == "s_nop" else 1
+        age = {r: a + step for r, a in age.items() if a + step < need}
+        dst = args.split(",")[0]
+        written = _sgprs(dst)
+        if op.startswith("v_"):
+            # (carry-out and compare results name their SGPR second or first)
+            if re.match(r"v_(add|sub|subrev|addc|subb|subbrev)_co_|v_div_scale|v_mad_[iu]64", op):
+                written |= _sgprs(args.split(",")[1])
+            age.update({r: 0 for r in written})
+        else:
+            for r in written:
+                age.pop(r, None)  # a scalar write: interlocked
+    return found
+
+
+def assembly(unit: str, tmp_path) -> str:
+    src, obj, extra = next(u for u in hip_build.UNITS if u[1] == unit)
+    out = tmp_path / (obj + ".s")
+    cmd = [hip_build.HIPCC, *hip_build.COMMON, *extra, "-x", "hip", "--cuda-device-only", "-S",
+           str(hip_build.CSRC / src), "-o", str(out)]
+    subprocess.run(cmd, check=True, capture_output=True, timeout=300)
+    return out.read_text()
+
+
+def test_the_scan_sees_a_short_wait():
+    short = "f:\n v_readlane_b32 s3, v1, 2\n s_mov_b32 m0, s9\n s_nop 0\n global_load_lds_dwordx4 v1, s[2:3]\n"
+    assert [n for n, _ in sgpr_hazards(short)] == [5]
+    assert not sgpr_hazards(short.replace("s_nop 0", "s_nop 3"))
+    assert not sgpr_hazards(short.replace("s_nop 0", "s_mov_b64 s[2:3], s[4:5]"))
+
+
+UNITS_WITH_ASM = ["sage_attn_keys.hip.o"]
+
+
+def test_only_these_units_load_in_inline_assembly():
+    """Vector memory instructions inside asm statements: the shared helper and
+    the keys-split kernels alone."""
+    hits = {p.name for p in hip_build.CSRC.iterdir()
+            if re.search(r'"(global|buffer|flat|scratch)_(load|store|atomic)', p.read_text())}
+    assert hits == {"sage_attn_keys.hip", "sage_attn_device.hpp"}, hits
+
+
+@pytest.mark.parametrize("unit", UNITS_WITH_ASM)
+def test_vector_memory_waits_for_its_base(unit, tmp_path):
+    asm = assembly(unit, tmp_path)
+    assert "global_load_lds_dwordx4" in asm
+    found = sgpr_hazards(asm)
+    assert not found, f"{unit}: SGPR read too soon after a vector write: {found[:8]}"
