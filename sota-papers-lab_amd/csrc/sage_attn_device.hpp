@@ -121,7 +121,7 @@ __device__ __forceinline__ void warm_l2(const uint8_t* kg, const uint8_t* vg, lo
             "s_mov_b32 m0, %0\n\t"
             "s_nop 0\n\t"
             "global_load_lds_dword %1, off" ::"s"(__builtin_amdgcn_readfirstlane((int)sink)), "v"(p)
-            : "memory", "m0");
+            : "memory");
 #endif
     }
 }

@@ -51,8 +51,10 @@ constexpr int KEY_ROWS = 32;  // queries a group
 // after a vector instruction wrote it, the compiler keeps no such distance to
 // an asm statement, and a base restored from a vector register's lanes
 // (v_readlane) arrives right before it. A scalar read of that SGPR is
-// interlocked, and a scalar write needs no wait before the load. (s_nop: one
-// wait state between M0's write, the copies' LDS base, and the load.)
+// interlocked, and a scalar write needs no wait before the load. M0, the copies'
+// LDS base, needs one wait state before the load (s_nop); it is a reserved
+// register that cannot be named as clobbered, so a kernel that uses these
+// helpers has no other use of it.
 // 4 KB, four copies of 64 lanes x 16 bytes: copy i reads base + 1024 i + even
 // (odd copies: + odd) and fills dst + 1024 i + 16 lane.
 __device__ __forceinline__ void copy_4k(const uint8_t* base, uint32_t even, uint32_t odd, uint32_t dst) {
@@ -68,7 +70,7 @@ __device__ __forceinline__ void copy_4k(const uint8_t* base, uint32_t even, uint
         "global_load_lds_dwordx4 %3, %0 offset:3072"
         : "=&s"(b)
         : "s"(__builtin_amdgcn_readfirstlane((int)dst)), "v"(even), "v"(odd), "s"(base)
-        : "memory", "m0");
+        : "memory");
 #endif
 }
 // 1 KB, 16 bytes a lane.
@@ -82,7 +84,7 @@ __device__ __forceinline__ void copy_1k(const uint8_t* base, uint32_t off, uint3
         "global_load_lds_dwordx4 %2, %0"
         : "=&s"(b)
         : "s"(__builtin_amdgcn_readfirstlane((int)dst)), "v"(off), "s"(base)
-        : "memory", "m0");
+        : "memory");
 #endif
 }
 // 256 bytes, four a lane.
@@ -96,7 +98,7 @@ __device__ __forceinline__ void copy_256(const uint8_t* base, uint32_t off, uint
         "global_load_lds_dword %2, %0"
         : "=&s"(b)
         : "s"(__builtin_amdgcn_readfirstlane((int)dst)), "v"(off), "s"(base)
-        : "memory", "m0");
+        : "memory");
 #endif
 }
 // At most N of the wave's vector memory operations are outstanding.

@@ -94,3 +94,16 @@ def test_vector_memory_waits_for_its_base(unit, tmp_path):
     assert "global_load_lds_dwordx4" in asm
     found = sgpr_hazards(asm)
     assert not found, f"{unit}: SGPR read too soon after a vector write: {found[:8]}"
+
+
+@pytest.mark.parametrize("unit", UNITS_WITH_ASM)
+def test_m0_belongs_to_the_asm_statements(unit, tmp_path):
+    """The copies write M0 (their LDS base) without the compiler's knowledge:
+    nothing it generates in the unit may hold a value there."""
+    inside, other = False, []
+    for n, line in enumerate(assembly(unit, tmp_path).splitlines(), 1):
+        if "ASMSTART" in line or "ASMEND" in line:
+            inside = "ASMSTART" in line
+        elif not inside and re.search(r"\bm0\b", line.split(";")[0]):
+            other.append((n, line.strip()))
+    assert not other, f"{unit}: M0 used outside the asm statements: {other[:8]}"
