@@ -65,7 +65,7 @@ namespace sage {
 // D/8 lanes hold a row, 8 channels a lane, 512/D rows at a time; rows past the
 // sequence are zeros. Its first half of iterations is the first 16-row group.
 template <int D>
-__device__ __forceinline__ void quantise_q(const uint16_t* __restrict__ q, int8_t* __restrict__ q8,
+__device__ __forceinline__ void quantise_q(const uint16_t* q, int8_t* __restrict__ q8,
                                            float* __restrict__ q_scale, const Geom& g, int q0, int lane,
                                            uint8_t* stage, v4i (&qa)[D / 32], float& qs) {
 #pragma clang fp contract(off)
@@ -167,14 +167,15 @@ __device__ __forceinline__ void quantise_q(const uint16_t* __restrict__ q, int8_
 // Workgroups a CU: four at head dim 64 (<= 128 VGPRs), three at head dim 128
 // (<= 168); the merged head-dim-128 kernel needs the registers of two.
 // QF (a forward call): the workgroup quantises its own queries (quantise_q)
-// instead of reading the prologue's codes.
+// instead of reading the prologue's codes, and the output may be those queries
+// themselves (q_readable_beside), so neither pointer is __restrict__.
 template <int D, bool CAUSAL, bool MERGE, bool QF>
-__global__ __launch_bounds__(256, D == 64 ? 4 : (MERGE ? 2 : 3)) void sage_attn(const uint16_t* __restrict__ q, int8_t* __restrict__ q8,
+__global__ __launch_bounds__(256, D == 64 ? 4 : (MERGE ? 2 : 3)) void sage_attn(const uint16_t* q, int8_t* __restrict__ q8,
                                                     float* __restrict__ q_scale,
                                                     const int8_t* __restrict__ k8,
                                                     const float* __restrict__ k_scale,
                                                     const uint8_t* __restrict__ v8, const float* __restrict__ stats,
-                                                    const float* __restrict__ kbias, uint16_t* __restrict__ out,
+                                                    const float* __restrict__ kbias, uint16_t* out,
                                                     Geom g) {
     constexpr int BN = ATTN_BN;
     constexpr int KS = D / 32;            // INT8 k-steps of 32 channels

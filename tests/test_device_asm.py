@@ -1,4 +1,4 @@
-"""The machine code of the kernels that carry inline assembly, on the CPU.
+"""What the compiler is told and what it makes of the device code, on the CPU.
 
 The compiler puts no wait states around an instruction inside an asm statement.
 On gfx9 a vector memory instruction may read an SGPR that a vector instruction
@@ -6,8 +6,11 @@ On gfx9 a vector memory instruction may read an SGPR that a vector instruction
 sooner it can see the old value, i.e. an address of two halves that do not
 belong together. A base pointer reaches such an asm straight from v_readlane
 whenever the register allocator parks SGPRs in lanes of a vector register, so
-the source alone does not show it: this test compiles the unit as the build
-does and reads the assembly."""
+the source alone does not show it: the test compiles the unit as the build
+does and reads the assembly.
+
+A forward call may write its output over Q, so the attention kernels that read
+the 16-bit queries promise no aliasing for neither of the two pointers."""
 from __future__ import annotations
 
 import re
@@ -61,10 +64,10 @@ def sgpr_hazards(asm: str, need: int = WAIT_STATES) -> list:
     return found
 
 
-def assembly(unit: str, tmp_path) -> str:
+def assembly(unit: str, tmp_path, *flags: str) -> str:
     src, obj, extra = next(u for u in hip_build.UNITS if u[1] == unit)
     out = tmp_path / (obj + ".s")
-    cmd = [hip_build.HIPCC, *hip_build.COMMON, *extra, "-x", "hip", "--cuda-device-only", "-S",
+    cmd = [hip_build.HIPCC, *hip_build.COMMON, *extra, "-x", "hip", "--cuda-device-only", "-S", *flags,
            str(hip_build.CSRC / src), "-o", str(out)]
     subprocess.run(cmd, check=True, capture_output=True, timeout=300)
     return out.read_text()
@@ -107,3 +110,19 @@ def test_m0_belongs_to_the_asm_statements(unit, tmp_path):
         elif not inside and re.search(r"\bm0\b", line.split(";")[0]):
             other.append((n, line.strip()))
     assert not other, f"{unit}: M0 used outside the asm statements: {other[:8]}"
+
+
+@pytest.mark.parametrize("unit", ["sage_attention.hip.o", "sage_attention_merged.hip.o"])
+def test_queries_and_output_may_alias(unit, tmp_path):
+    """sage_attn<D, CAUSAL, MERGE, QF = true>(q, ..., out, geometry): the host
+    launches it with out = q (q_readable_beside)."""
+    ir = assembly(unit, tmp_path, "-emit-llvm", "-Xclang", "-disable-llvm-passes")
+    seen = 0
+    for args in re.findall(r"define [^@\n]*@_ZN4sage9sage_attnILi\d+ELb[01]ELb[01]ELb1EE\w*\(([^\n]*?)\) #", ir):
+        ptrs = [a for a in args.split(", ") if "ptr" in a and "byref" not in a]
+        assert len(ptrs) == 9, args
+        for which in (0, 8):
+            assert "noalias" not in ptrs[which], (which, ptrs[which])
+        assert all("noalias" in p for p in ptrs[3:8])  # codes, scales and statistics: read only
+        seen += 1
+    assert seen == (2 if "merged" in unit else 4)
