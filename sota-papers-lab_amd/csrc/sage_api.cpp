@@ -7,12 +7,14 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
 #include <new>
 #include <string>
+#include <utility>
 
 #include "sage_device.hpp"
 #include "sage_internal.hpp"
@@ -569,15 +571,33 @@ sage_status attend_view(const sage_attention* s, const WsView& w, const Geom& ge
     return r == SAGE_OK ? launch_attend(s, w, geom, out, nullptr) : r;
 }
 
+// Whether the rows of a [batch][token][head] view of `d` channels are known to
+// share no element: each stride, in rising order, steps over all that the
+// smaller ones span.
+static bool rows_apart(const sage_strides& st, const sage_shape& sh, uint64_t d) {
+    std::pair<uint64_t, uint64_t> dims[3] = {{st.batch, sh.batch}, {st.token, sh.tokens}, {st.head, sh.heads}};
+    std::sort(dims, dims + 3);
+    uint64_t span = d;
+    for (const auto& [stride, count] : dims) {
+        if (count == 1) continue;
+        uint64_t step;
+        if (stride < span || __builtin_mul_overflow(stride, count - 1, &step) ||
+            __builtin_add_overflow(span, step, &span))
+            return false;
+    }
+    return true;
+}
+
 // Whether the attention kernel may read Q while it writes `out`: it reads each
 // workgroup's query rows before it writes the same rows, so the two views are
-// the same or apart.
-static bool q_readable_beside(const sage_attention* s, const sage_plan& plan, const sage_tensor* q,
-                              const sage_tensor_mut* out) {
+// apart, or the same with no row shared by two queries (a Q broadcast over
+// heads or batch items is read by workgroups that start after others wrote it).
+bool q_readable_beside(uint64_t d, const sage_shape& shape, const sage_tensor* q, const sage_tensor_mut* out) {
     const sage_strides &a = q->strides, &b = out->strides;
-    if (q->data == out->data && a.batch == b.batch && a.token == b.token && a.head == b.head) return true;
-    const uint64_t nq = 2 * sage_strides_extent(&a, plan.shape.batch, plan.shape.tokens, plan.shape.heads, s->head_dim);
-    const uint64_t no = 2 * sage_strides_extent(&b, plan.shape.batch, plan.shape.tokens, plan.shape.heads, s->head_dim);
+    if (q->data == out->data && a.batch == b.batch && a.token == b.token && a.head == b.head)
+        return rows_apart(a, shape, d);
+    const uint64_t nq = 2 * sage_strides_extent(&a, shape.batch, shape.tokens, shape.heads, d);
+    const uint64_t no = 2 * sage_strides_extent(&b, shape.batch, shape.tokens, shape.heads, d);
     const uintptr_t pq = reinterpret_cast<uintptr_t>(q->data), po = reinterpret_cast<uintptr_t>(out->data);
     return pq + nq <= po || po + no <= pq;
 }
@@ -594,7 +614,7 @@ sage_status forward_view(const sage_attention* s, const WsView& w, const sage_te
     Geom probe = g;
     if (s->config.tile.warps == 8) probe.flags |= F_WAVES8;
     const bool later = attention_quantises_q((int)s->head_dim, probe) && attend_check(s, w, out) == SAGE_OK &&
-                       q_readable_beside(s, w.plan, q, out);
+                       q_readable_beside(s->head_dim, w.plan.shape, q, out);
     Geom run = g;
     if (later) run.flags |= F_Q_LATER;
     r = launch_prepare(s, w, q, k, v, opts, run, nullptr);

@@ -124,6 +124,8 @@ sage_status workspace_layout(const sage_attention* s, const sage_shape* shape, c
 sage_status prepare_view(const sage_attention* s, const WsView& w, const sage_tensor* q, const sage_tensor* k,
                          const sage_tensor* v, const sage_options* opts, Geom* geom, const QkvDev* qa);
 sage_status attend_view(const sage_attention* s, const WsView& w, const Geom& geom, const sage_tensor_mut* out);
+// Whether Q may be read by the kernel that writes `out`.
+bool q_readable_beside(uint64_t head_dim, const sage_shape& shape, const sage_tensor* q, const sage_tensor_mut* out);
 // prepare_view then attend_view in one call: where the whole-key kernel runs,
 // Q's codes are left to it.
 sage_status forward_view(const sage_attention* s, const WsView& w, const sage_tensor* q, const sage_tensor* k,

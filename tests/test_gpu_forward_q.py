@@ -88,6 +88,25 @@ def test_output_over_q(oracle, torch_gpu, d, where):
     assert np.array_equal(from_device16(out), from_device16(o))
 
 
+@pytest.mark.parametrize("d", [64, 128])
+def test_output_over_a_broadcast_q(oracle, torch_gpu, d):
+    """One query row a token, broadcast over the heads of one KV head, and the
+    output over it: every head's result is the same row, from the Q of before
+    the call."""
+    torch = torch_gpu
+    h = 475 if d == 64 else 240
+    S, p, sa, ws, ts, opts = _setup(torch, oracle, 1, h, 130, d, dict(kv_heads=1), "bthd")
+    q = ts[0][:, :, :1].contiguous()
+    want = torch.empty_like(ts[0])
+    st = S.Strides(130 * d, d, 0)
+    sa.prepare(ws, S.Tensor(q, st), S.Tensor(ts[1]), S.Tensor(ts[2]), opts)
+    sa.attend(ws, S.TensorMut(want))
+    sa.forward(ws, S.Tensor(q, st), S.Tensor(ts[1]), S.Tensor(ts[2]), S.TensorMut(q, st), opts)
+    torch.cuda.synchronize()
+    assert np.array_equal(from_device16(q)[:, :, 0], from_device16(want)[:, :, 0])
+    assert np.array_equal(from_device16(want)[:, :, -1], from_device16(want)[:, :, 0])
+
+
 def test_refused_output_leaves_a_prepared_workspace(oracle, torch_gpu):
     """An output that attend refuses: forward reports attend's text, and the
     workspace holds prepare's codes, as after the two calls."""

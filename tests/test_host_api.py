@@ -261,3 +261,45 @@ def test_rope_tables_match_the_oracle(S, oracle, d):
     with pytest.raises(S.SageError, match="RoPE table: buffer holds 10 elements, needs"):
         _check = S._check
         _check(S.lib().sage_rope_table(0, d, 2, 2, 1, 100.0, out.ctypes.data, out.size))
+
+
+# (shape, Q strides, output strides, output's offset in elements), head dim 64
+Q_BESIDE = [
+    ((2, 3, 5), (960, 192, 64), (960, 192, 64), 0),          # in place
+    ((2, 3, 5), (960, 64, 320), (960, 64, 320), 0),          # in place, head-major
+    ((2, 3, 5), (2880, 576, 64), (2880, 576, 64), 0),        # in place in a packed projection
+    ((2, 3, 5), (960, 192, 64), (960, 192, 64), 1920),       # apart
+    ((2, 3, 5), (960, 192, 64), (960, 192, 64), 64),         # one head on
+    ((2, 3, 5), (960, 192, 64), (960, 64, 320), 0),          # other strides over the same memory
+    ((1, 3, 5), (0, 192, 64), (0, 192, 64), 0),              # a stride that is never taken
+    ((2, 3, 5), (320, 64, 0), (320, 64, 0), 0),              # Q and output broadcast over heads
+    ((2, 3, 5), (0, 192, 64), (0, 192, 64), 0),              # over batch items
+    ((2, 3, 5), (960, 128, 64), (960, 128, 64), 0),          # heads of one token in the next one's
+    ((2, 3, 5), (960, 192, 32), (960, 192, 32), 0),          # rows half in each other
+    ((2, 2, 2), (64, 256, 128), (64, 256, 128), 0),          # batch items between the heads
+]
+
+
+@pytest.mark.parametrize("shape,qs,os_,off", Q_BESIDE)
+def test_queries_read_beside_the_output(S, shape, qs, os_, off):
+    """The attention kernel reads a workgroup's query rows, writes the same
+    rows of the output and runs beside workgroups that do the same, so a forward
+    call leaves Q to it only where no output row touches another query's row
+    (here by every pair of rows)."""
+    from spl_sage import _abi
+
+    b, h, n = shape
+    f = _abi.lib()._ZN4sage17q_readable_besideEmRK10sage_shapePK11sage_tensorPK15sage_tensor_mut
+    f.restype = C.c_bool
+    base, d = 1 << 20, 64
+    q = _abi.sage_tensor(base, 1 << 30, qs, 0)
+    o = _abi.sage_tensor_mut(base + 2 * off, 1 << 30, os_, 0)
+    got = f(C.c_uint64(d), C.byref(_abi.sage_shape(b, h, n, h)), C.byref(q), C.byref(o))
+    rows = [(i, t, j) for i in range(b) for t in range(n) for j in range(h)]
+    at = lambda r, s, o: o + sum(x * y for x, y in zip(r, s))  # noqa: E731
+    safe = all(abs(at(r, qs, 0) - at(w, os_, off)) >= d for r in rows for w in rows if r != w)
+    assert safe or not got  # never where a row is overwritten before its reader
+    if qs == os_ and off == 0:
+        assert got == safe
+    elif off >= 1920:
+        assert got
