@@ -502,8 +502,15 @@ class SageAttention:
                 opts: Optional[Options] = None) -> None:
         """prepare, then attend, as one call."""
         o = (opts or Options())._c()
-        _check(lib().sage_forward(self._h, ws._h, C.byref(q._c()), C.byref(k._c()), C.byref(v._c()),
-                                  C.byref(out._c()), C.byref(o)))
+        qc, kc, vc = q._c(), k._c(), v._c()
+        try:
+            oc = out._c()
+        except Exception:
+            # An output that is no 16-bit tensor is attend's refusal: prepare
+            # has run by then (and its own refusals come first).
+            self.prepare(ws, q, k, v, opts)
+            raise
+        _check(lib().sage_forward(self._h, ws._h, C.byref(qc), C.byref(kc), C.byref(vc), C.byref(oc), C.byref(o)))
 
     def prepare_qkv(self, ws: Workspace, input, norm=None, rope=None, opts: Optional[Options] = None) -> None:
         """prepare fed straight from the fused QKV projection (spl_sage.qkv)."""

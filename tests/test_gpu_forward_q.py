@@ -116,6 +116,25 @@ def test_refused_output_leaves_a_prepared_workspace(oracle, torch_gpu):
     short = torch.empty(64, dtype=ts[0].dtype, device="cuda")
     with pytest.raises(S.SageError, match="output holds 64 elements"):
         sa.forward(ws, *tens, S.TensorMut(short, S.Strides.bthd(1000, 58, 64)), opts)
+    _check_left_prepared(S, torch, sa, ws, ts, tens, opts)
+
+
+def test_output_of_another_type_leaves_a_prepared_workspace(oracle, torch_gpu):
+    """The same for an output that the Python layer refuses; a bad Q is still
+    the first refusal."""
+    torch = torch_gpu
+    S, p, sa, ws, ts, opts = _setup(torch, oracle, 1, 58, 1000, 64, {}, "bthd")
+    tens = [S.Tensor(t) for t in ts]
+    f32 = torch.empty(ts[0].shape, dtype=torch.float32, device="cuda")
+    with pytest.raises(S.SageError, match="Q holds 64 elements"):
+        sa.forward(ws, S.Tensor(f32.to(ts[0].dtype)[0, 0, 0].clone(), S.Strides.bthd(1000, 58, 64)), *tens[1:],
+                   S.TensorMut(f32), opts)
+    with pytest.raises(S.SageError, match="sage tensors are bf16 or fp16"):
+        sa.forward(ws, *tens, S.TensorMut(f32), opts)
+    _check_left_prepared(S, torch, sa, ws, ts, tens, opts)
+
+
+def _check_left_prepared(S, torch, sa, ws, ts, tens, opts):
     o1, o2 = torch.empty_like(ts[0]), torch.empty_like(ts[0])
     sa.attend(ws, S.TensorMut(o1))
     sa.forward(ws, *tens, S.TensorMut(o2), opts)
