@@ -622,7 +622,7 @@ sage_status forward_view(const sage_attention* s, const WsView& w, const sage_te
     *geom = g;
     *prepared = !later;
     r = attend_check(s, w, out);
-    if (r == SAGE_OK) r = launch_attend(s, w, run, out, q->data);
+    if (r == SAGE_OK) r = launch_attend(s, w, run, out, later ? q->data : nullptr);
     if (r == SAGE_OK) *prepared = true;
     return r;
 }
