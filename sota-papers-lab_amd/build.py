@@ -54,17 +54,25 @@ UNITS = [
 ]
 
 
-def _compile(unit) -> Path:
-    src, obj, extra = unit
-    out = OBJ / obj
-    lang = ["-x", "hip"] if src.endswith(".hip") else []
-    cmd = [HIPCC, *COMMON, *extra, *lang, "-c", str(CSRC / src), "-o", str(out)]
-    res = subprocess.run(cmd, capture_output=True, text=True)
+def _run(cmd, what: str) -> str:
+    """Runs one step; returns what it wrote to stderr. A failure names the step,
+    its exit status (a compiler killed from outside writes nothing) and its
+    command."""
+    res = subprocess.run(cmd, capture_output=True, text=True, errors="replace")
     # hipcc's host pass does not know the packed-fp32 feature and says so; that is harmless.
     noise = "'-packed-fp32-ops' is not a recognized feature"
     err = "\n".join(l for l in res.stderr.splitlines() if noise not in l)
     if res.returncode != 0:
-        raise RuntimeError(f"hipcc failed for {obj}:\n{err}")
+        how = f"killed by signal {-res.returncode}" if res.returncode < 0 else f"exit status {res.returncode}"
+        raise RuntimeError(f"{what} failed ({how}): {' '.join(cmd)}\n{res.stdout}{err}")
+    return err
+
+
+def _compile(unit) -> Path:
+    src, obj, extra = unit
+    out = OBJ / obj
+    lang = ["-x", "hip"] if src.endswith(".hip") else []
+    err = _run([HIPCC, *COMMON, *extra, *lang, "-c", str(CSRC / src), "-o", str(out)], f"compiling {obj}")
     if err.strip():
         print(err, file=sys.stderr)
     return out
@@ -77,9 +85,7 @@ def build(verbose: bool = True) -> Path:
         objs = list(ex.map(_compile, UNITS))
     tmp = LIB.with_suffix(".so.tmp")
     cmd = [HIPCC, "-shared", f"--offload-arch={ARCH}", "-fPIC", *map(str, objs), "-o", str(tmp)]
-    res = subprocess.run(cmd, capture_output=True, text=True)
-    if res.returncode != 0:
-        raise RuntimeError(f"link failed:\n{res.stderr}")
+    _run(cmd, f"linking {LIB.name}")
     # Every kernel the launchers name must be in the library: load it with all
     # symbols resolved now (a kernel the host pass failed to instantiate shows
     # up here, not at first use on a GPU box).

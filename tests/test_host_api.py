@@ -303,3 +303,18 @@ def test_queries_read_beside_the_output(S, shape, qs, os_, off):
         assert got == safe
     elif off >= 1920:
         assert got
+
+
+@pytest.mark.parametrize("script,says", [("kill -9 $$", "killed by signal 9"), ("echo why >&2; exit 3", "exit status 3")])
+def test_a_failed_build_step_says_how(tmp_path, monkeypatch, script, says):
+    """A compiler that is killed writes nothing: the step and its status are
+    named all the same."""
+    import build as hip_build
+
+    cc = tmp_path / "hipcc"
+    cc.write_text(f"#!/bin/sh\n{script}\n")
+    cc.chmod(0o755)
+    monkeypatch.setattr(hip_build, "HIPCC", str(cc))
+    monkeypatch.setattr(hip_build, "OBJ", tmp_path)
+    with pytest.raises(RuntimeError, match=rf"compiling sage_api.cpp.o failed \({says}\)"):
+        hip_build._compile(("sage_api.cpp", "sage_api.cpp.o", []))
