@@ -934,55 +934,90 @@ static hipError_t resources_of(int head_dim, int* regs, int* spill, int* lds) {
 // default order and are built in the second pass.
 #ifndef SAGE_ATTN_MERGED
 
-// How the keys are split (KeySplit), by the number n of 128-query tiles and
-// their remainder r over whole multiples of the chip's 256 CUs.
+// How the keys are split (KeySplit), by the number n of 128-query tiles, their
+// remainder r over whole multiples of the chip's 256 CUs, and the 64-key blocks.
 //
 // Few tiles. A tile is one wave a SIMD, and a lone wave takes 1.6 times the
-// chip's best time a block, so up to about n = 256 the chip is short of waves
-// however long the keys; four or two shares make more of them, but read K and V
-// once per 32 queries instead of 128 and sweep the keys' first shares twice (20
-// to 35% slower on a full chip). Measured (us, whole keys / four / two shares):
-//   D 64        96 tiles N 689: 11.8 / 8.0 / 9.1     176, N 1378: 19.9 / 16.7 / 19.0
-//               216, N 1100: 18.2 / 17.9             256, N 1000: 17.3 / 17.2 / 17.1
-//   D 64 causal 256, N 1000: 16.3 / 11.5 / 12.9      352, N 2756: 36.2 / 27.6 / 28.6
-//               480, N 5000: 81.3 / 67.8 / 63.2      512, N 1000: 18.4 / 22.1 / 18.9
-//   D 128       128, N 8192: 118 / 76.9 / 84.7       176, N 1378: 27.6 / 27.5 / 27.8
-//   D 128 causal 176, N 1378: 26.8 / 20.7 / 21.2     256, N 1000: 22.3 / 21.5 / 18.9
-//               352, N 2756: 49.3 / 47.7 / 43.9      384, N 689: 18.0 / 24.5 / 21.8
-//               320, N 1000: 23.2 / - / 25.4         (whole tiles in sage_attn's paired order)
-//   merged      D 64 96 tiles, stride 2: 7.2 / 6.2 / 6.4, stride 4: 5.5 / 5.7 / 5.3;
-//               D 128 96, stride 2: 9.8 / 8.6 / 8.7, stride 4: 8.2 / 8.2 / 7.1;
-//               352 D 64: 21.9 / 23.4 / 21.9, D 128: 29.8 / 41.5 / 37.9
-// (A causal tile's keys end at its queries, so causal grids carry half the
-// work and longer tails.)
+// chip's best time a block, so up to about n = 256 the chip is short of waves;
+// four or two shares make more of them, but read K and V once per 32 queries
+// instead of 128, sweep the keys' first shares twice, and leave Q's codes to
+// the prologue. They pay while their workgroups are resident at once (four a
+// CU at head dim 64, two at 128: 256 and 128 tiles of four shares) and, where
+// the keys are long enough for the loop to outweigh the rest, a little beyond.
+// A forward on the GPU, us, whole keys / split (graph replays, one box):
+//   D 64        96 tiles N 684: 23.5 / 18.4          192, N 100: 17.8 / 18.3   192, N 1000: 27.6 / 25.0
+//               224, N 484: 22.9 / 23.3              224, N 2020: 39.4 / 38.6  256, N 1000: 28.5 / 28.1
+//   D 128       128, N 100: 23.3 / 21.6              144, N 100: 24.3 / 28.0   128, N 4068: 80.6 / 56.8
+//               144, N 1000: 37.1 / 38.3             160, N 2020: 53.9 / 52.8  160, N 4068: 82.1 / 77.9
+// A causal tile's keys end at its queries, so causal grids carry half the work
+// and longer tails (whole / two shares / four):
+//   D 64        160, N 356: 21.3 / 20.3 / 19.8       222: 21.6 / 20.7 / 21.6   320, N 740: 31.3 / 28.4 / 30.9
+//               400, N 740: 31.4 / 32.7 / 33.5       400, N 1000: 37.5 / 38.9 / 35.0
+//               440, N 2532: 58.1 / 56.6 / 53.7      480, N 2532: 50.9 / 50.8 / 51.0
+//               480, N 3044: 62.1 / 65.6 / 63.6      480, N 4068: 87.9 / 77.8 / 76.0
+//   D 128       126, N 356: 27.7 / 24.7 / 23.9       159: 29.3 / 28.9 / 30.4   204, N 740: 36.1 / 36.1 / 38.1
+//               208, N 1636: 48.8 / 43.4 / 43.2      248, N 1000: 40.0 / 39.3 / 43.0
+//               288, N 484: 36.7 / 40.9 / 42.7       288, N 2020: 70.8 / 63.7 / 66.3
+//               352, N 2764: 70.8 / 66.1 / 72.8      352, N 1000: 51.6 / 53.6 / 54.6
+// With fewer than five heads an XCD's range lies within one head, whose long
+// tiles are all its work, so there the line is where the XCDs hold every
+// workgroup at once or little more:
+//   D 64 480, 2 heads (29412 keys) 415 / 457 / 418, 3 heads 279 / 280 / 297;
+//   D 128 252, 4 heads 136 / 113 / 116; 278, 2 heads 297 / 379 / 304; 284, 4 heads 155 / 169 / 156.
+// Merged (whole / two shares):
+//   D 64        222, stride 2, 1 frame: 24.3 / 24.0  220, 8 frames: 49.9 / 45.5
+//               176, stride 4, 8 frames: 40.6 / 39.2 222, stride 4, 1 frame: 32.4 / 35.2
+//   D 128       120, stride 2, 1 frame: 34.7 / 30.8  170, 3 frames: 45.8 / 47.0
+//               102, stride 4, 3 frames: 48.6 / 46.1 120, 1 frame: 45.3 / 49.2
 //
 // A few tiles over. Whole tiles alone give r CUs one tile more than the rest,
 // and those set the time. Left whole beside the others split into four
-// workgroups each, the remainder spreads over all CUs (us, all whole / r split):
-//   D 64  r 8 over 256, N 1000: 23.3 / 17.0   96, N 2756: 52.5 / 37.4   128, N 2048: 38.8 / 29.8
-//         186, N 4300: 79.1 / 72.8            224, N 5000: 85.1 / 90.5
-//         44 over 512, N 17776: 354 / 293     128, N 1000: 31.8 / 27.6  160, N 1000: 31.6 / 31.7
-//         64 over 768, N 1000: 39.1 / 34.6    123, N 12600: 334 / 303
-//         74 over 1024, N 15500: 498 / 447    84 over 1280, N 15800: 597 / 568   64 over 1536: 66.9 / 61.9
-//   D 128 8 over 256, N 1000: 30.9 / 25.5     96, N 2756: 63.5 / 59.8   128, N 2048: 50.9 / 49.9
-//         44 over 512, N 17776: 483 / 423     64, N 1000: 44.9 / 39.0   96, N 1000: 45.2 / 45.2
-//         64 over 768, N 1000: 59.8 / 52.3    74 over 1024, N 15500: 690 / 672   16 over 1280: 82.6 / 76.3
-// (A forward call's Q codes cost 2% more outside sage_attn, so gains below
-// that are left.) The tile of the context's Config does not matter here: it
-// picks a layout, never a result.
-static KeySplit key_split(int head_dim, const Geom& g) {
-    const long long n = (long long)g.q_tiles * g.heads * g.batch;
-    if (g.merge > 1) return {n <= (head_dim == 64 ? 224 : 128) ? 2 : 0, 0};
-    if (g.flags & F_CAUSAL) {
-        if (head_dim == 64) return {n <= 320 ? 4 : n <= 480 ? 2 : 0, 0};
-        return {n <= 208 ? 4 : n <= 288 ? 2 : 0, 0};
+// workgroups each, the remainder spreads over all CUs. Its own limit is
+// residency again (three workgroups a CU at head dim 128: 64 split tiles beside
+// 512 whole ones); short keys, and more whole tiles a CU, leave it less to gain
+// (whole / r split):
+//   D 64  r 64 over 256, N 100: 22.0 / 21.7   144, N 100: 23.5 / 24.9   176, N 484: 30.5 / 30.1   128, N 3044: 68.9 / 59.2
+//         64 over 512, N 228: 30.8 / 30.2     128, N 484: 37.4 / 37.3   128, N 1000: 47.8 / 45.6
+//         32 over 768, N 228: 38.2 / 38.3     64, N 484: 45.7 / 45.2    112, N 996: 58.4 / 58.6   108, N 1508: 73.2 / 72.0
+//         64 over 1024, N 484: 54.6 / 54.3    80, N 1508: 87.6 / 86.8
+//         72 over 1280, N 1000: 81.7 / 83.2   64, N 1508: 102.4 / 100.8 64 over 1536, N 1000: 92.2 / 93.4, 2020: 139.6 / 137.2
+//   D 128 r 64 over 256, N 100: 32.8 / 31.4   88, N 1000: 50.6 / 51.0   80, N 10724: 231 / 217   104, N 3044: 92.7 / 93.8
+//         32 over 512, N 484: 56.3 / 56.7     64, N 1000: 69.6 / 68.5   72, N 1000: 69.5 / 73.4   64, N 3044: 124.7 / 117.1
+//         32 over 768, N 484: 74.5 / 75.1     64, N 1000: 91.3 / 90.5   80, N 1000: 91.8 / 97.2   48, N 3044: 167 / 153
+//         32 over 1024, N 2020: 153.9 / 156.2 32, N 3044: 200.5 / 197.2 56, N 3044: 200.6 / 201.3
+//         16 over 1280, N 3044: 234.0 / 228.5 64 over 1536, N 5092: 404 / 396 (runs of one side differ by 8%)
+// The tile of the context's Config does not matter here: it picks a layout,
+// never a result.
+KeySplit key_split(int head_dim, long long n, int heads, int kblocks, int merge, bool causal) {
+    const bool wide = head_dim == 128;
+    if (merge > 1) return {n <= (wide ? (merge == 2 ? 128 : 104) : (merge == 2 ? 224 : 176)) ? 2 : 0, 0};
+    if (causal && !wide) {
+        if (kblocks < 16) return {n <= 176 ? 4 : n <= 320 ? 2 : 0, 0};
+        return {n <= (kblocks >= 56 && heads >= 5 ? 480 : 448) ? 4 : 0, 0};
     }
-    if (n <= (head_dim == 64 ? 224 : 160)) return {4, 0};
-    // The largest remainder that is split beside 1, 2, .. tiles a CU.
-    static constexpr int MOST[2][6] = {{176, 136, 112, 80, 80, 64}, {96, 72, 80, 48, 32, 0}};
+    if (causal) {
+        if (kblocks < 16) return {n <= 128 ? 4 : 0, 0};
+        return {n <= 208 ? 4 : n <= (heads >= 5 ? 288 : 256) ? 2 : 0, 0};
+    }
+    if (n <= (wide ? (kblocks >= 32 ? 160 : 128) : (kblocks >= 16 ? 224 : 192))) return {4, 0};
     const long long f = n / 256, r = n % 256;
-    if (f >= 1 && f <= 6 && r > 0 && r <= MOST[head_dim == 128][f - 1]) return {4, (int)(n - r)};
+    if (f == 0 || f > 6 || r == 0) return {0, 0};
+    // [whole tiles a CU - 1]: the largest remainder that is split from so many
+    // key blocks on, for shorter keys and longer ones.
+    struct Line {
+        int most, blocks;
+    };
+    static constexpr Line LINES[2][6][2] = {
+        {{{64, 1}, {176, 8}}, {{64, 1}, {136, 8}}, {{80, 8}, {112, 24}}, {{64, 8}, {80, 24}}, {{0, 0}, {80, 24}}, {{0, 0}, {64, 32}}},
+        {{{64, 1}, {96, 48}}, {{64, 16}, {64, 16}}, {{64, 16}, {64, 16}}, {{0, 0}, {32, 48}}, {{0, 0}, {32, 48}}, {{0, 0}, {0, 0}}}};
+    for (const Line& l : LINES[wide][f - 1])
+        if (r <= l.most && kblocks >= l.blocks) return {4, (int)(n - r)};
     return {0, 0};
+}
+
+static KeySplit key_split(int head_dim, const Geom& g) {
+    return key_split(head_dim, (long long)g.q_tiles * g.heads * g.batch, g.heads * g.batch, g.kblocks, g.merge,
+                     g.flags & F_CAUSAL);
 }
 
 // The whole-key four-wave kernels have the variant; the sage options' QK

@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 from conftest import from_device16, to_device16
+from sage_gpu_helpers import split_of
 
 pytestmark = pytest.mark.gpu
 
@@ -43,6 +44,7 @@ def _setup(torch, oracle, b, h, n, d, kw, layout):
         ts = [to_device16(torch, np.ascontiguousarray(x.transpose(0, 2, 1, 3)), p.dtype).transpose(1, 2) for x in (q, k, v)]
     else:
         ts = [to_device16(torch, x, p.dtype) for x in (q, k, v)]
+    assert split_of(p)[0] == 0, "a grid of the keys-split kernels: Q stays with the prologue"
     sa = S.SageAttention(None, d)
     merge = S.KvMerge.Dense if p.merge == 1 else S.KvMerge.Pool(p.merge, S.FrameLayout(*p.layout))
     ws = sa.workspace(S.Shape(b, h, n, p.kv_heads), merge)

@@ -16,7 +16,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from sage_gpu_helpers import run, sample_rows
+from sage_gpu_helpers import run, sample_rows, split_of
 from test_gpu_fuzz import _check
 
 pytestmark = pytest.mark.gpu
@@ -32,14 +32,15 @@ SPLIT = [
     (1, 5, 7000, 64, dict(dtype=1)),                     # 275 tiles: uneven XCD ranges
     (2, 33, 1003, 64, dict(kv_heads=11)),                # 512 whole, 16 split
     (1, 5, 6700, 128, {}),                               # 265: one buffer a wave
-    (3, 30, 700, 128, dict(dtype=1)),                    # 512 whole, 28 split
+    (2, 34, 1003, 128, dict(dtype=1)),                   # 512 whole, 32 split
     (1, 2, 4170, 128, dict(causal=True)),
     (3, 4, 700, 64, dict(kv_heads=2, causal=True)),
     (1, 8, 1000, 64, dict(causal=True)),                 # dealt longest first
-    (1, 48, 1100, 64, dict(causal=True, dtype=1)),       # two shares (432 tiles)
+    (1, 48, 700, 64, dict(causal=True)),                 # two shares (288 tiles of short keys)
+    (1, 48, 1100, 64, dict(causal=True, dtype=1)),       # 432 tiles
     (1, 32, 1050, 128, dict(kv_heads=4, causal=True)),   # two shares (288 tiles)
     (1, 3, 3 * 95, 64, dict(merge=2, layout=(3, 5, 9, 10, 1))),
-    (2, 2, 50 * 95, 128, dict(merge=4, layout=(50, 5, 9, 10, 0))),
+    (1, 2, 50 * 95, 128, dict(merge=4, layout=(50, 5, 9, 10, 0))),
 ]
 WHOLE = [
     (1, 58, 1000, 64, {}),
@@ -63,6 +64,7 @@ def _problem(oracle, b, h, n, d, kw, seed):
 @pytest.mark.parametrize("b,h,n,d,kw", SPLIT + WHOLE, ids=[f"b{c[0]}h{c[1]}n{c[2]}d{c[3]}" for c in SPLIT + WHOLE])
 def test_against_reference_arithmetic(oracle, torch_gpu, b, h, n, d, kw):
     p, q, k, v = _problem(oracle, b, h, n, d, kw, 100 + n + d)
+    assert (split_of(p)[0] > 0) == ((b, h, n, d, kw) in SPLIT)
     _, o = run(torch_gpu, p, q, k, v, want_ws=False)
     rows = sample_rows(n, max(8, 4096 // (b * h)), seed=n)
     _check(oracle, p, oracle.prologue(p, q, k, v), o, rows, q, k, v, p.dtype, f"b{b} h{h} n{n} d{d} {kw}")
@@ -74,6 +76,7 @@ def test_eight_waves_equal_four_over_the_line(oracle, torch_gpu, b, h, n, d, kw)
     import spl_sage as S
 
     p, q, k, v = _problem(oracle, b, h, n, d, kw, 200 + n)
+    assert split_of(p)[0] == 0
     _, base = run(torch_gpu, p, q, k, v, want_ws=False)
     _, o = run(torch_gpu, p, q, k, v, want_ws=False, tile=S.Tile(8, 1, 3))
     assert np.array_equal(o, base)

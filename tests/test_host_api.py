@@ -318,3 +318,55 @@ def test_a_failed_build_step_says_how(tmp_path, monkeypatch, script, says):
     monkeypatch.setattr(hip_build, "OBJ", tmp_path)
     with pytest.raises(RuntimeError, match=rf"compiling sage_api.cpp.o failed \({says}\)"):
         hip_build._compile(("sage_api.cpp", "sage_api.cpp.o", []))
+
+
+# (head dim, tiles, heads, key blocks, merge stride, causal) -> (shares, whole):
+# both sides of lines where the other kernel took longer.
+SPLITS = [
+    ((128, 278, 2, 278, 1, True), (0, 0)),     # few heads of long keys: two shares 379 us, whole keys 297
+    ((128, 252, 4, 126, 1, True), (2, 0)),
+    ((128, 288, 18, 32, 1, True), (2, 0)),
+    ((128, 288, 72, 8, 1, True), (0, 0)),      # short keys: 40.9, 36.7
+    ((64, 460, 2, 460, 1, True), (0, 0)),      # 457, 415
+    ((64, 480, 15, 64, 1, True), (4, 0)),
+    ((64, 288, 48, 12, 1, True), (2, 0)),
+    ((128, 144, 144, 2, 1, False), (0, 0)),    # 28.0, 24.3
+    ((128, 160, 5, 64, 1, False), (4, 0)),
+    ((128, 584, 73, 16, 1, False), (0, 0)),    # 73.3, 69.1: over three workgroups a CU
+    ((128, 576, 72, 16, 1, False), (4, 512)),
+    ((128, 580, 290, 4, 1, False), (0, 0)),    # 56.0, 49.9
+    ((64, 1060, 530, 4, 1, False), (0, 0)),
+    ((64, 352, 16, 44, 1, False), (4, 256)),
+    ((64, 640, 80, 16, 1, False), (4, 512)),   # 47.8, 45.6
+    ((64, 880, 110, 16, 1, False), (0, 0)),    # 58.6, 58.4
+    ((64, 876, 73, 24, 1, False), (4, 768)),   # 72.0, 73.2
+    ((128, 344, 43, 16, 1, False), (0, 0)),    # 51.0, 50.6
+    ((128, 336, 4, 168, 1, False), (4, 256)),  # 231, 217
+    ((128, 120, 20, 4, 4, False), (0, 0)),     # merged, stride 4: 49.2, 45.3
+    ((64, 222, 37, 2, 4, False), (0, 0)),      # 35.2, 32.4
+    ((64, 222, 37, 4, 2, False), (2, 0)),
+]
+
+
+@pytest.mark.parametrize("args,want", SPLITS)
+def test_key_split_lines(S, args, want):
+    from sage_gpu_helpers import key_split
+
+    assert key_split(*args) == want
+
+
+def test_key_split_gives_what_the_kernels_are_built_for(S):
+    """Merged plans two shares, dense ones four (alone or beside a whole number
+    of tiles a CU with a remainder), causal ones four or two."""
+    from sage_gpu_helpers import key_split
+
+    for d in (64, 128):
+        for tiles in [*range(1, 2100), 1 << 20, 1 << 34]:
+            for heads in (1, 4, 5, 64):
+                for kb in (1, 4, 8, 16, 24, 32, 48, 56, 300):
+                    s, w = key_split(d, tiles, heads, kb, 1, False)
+                    assert (s, w) == (0, 0) or (s == 4 and w % 256 == 0 and w < tiles and (w or tiles < 256)), (d, tiles)
+                    s, w = key_split(d, tiles, heads, kb, 1, True)
+                    assert s in (0, 2, 4) and w == 0
+            for m in (2, 4):
+                assert key_split(d, tiles, 4, 8, m, False) in ((0, 0), (2, 0))
