@@ -571,6 +571,8 @@ __device__ __forceinline__ void put_v(uint8_t* vt, int ch, int kl, const float* 
 // Under QK LayerNorm (LN) each K row (each member, when merging) is
 // normalised before it is summed (sage_quant.cu:271).
 //
+// MERGE is the merge stride, or 0 for plain plans (the fused projection's
+// gather walks members one by one and has one instantiation, 4, for both).
 // Merged plans have instantiations of their own: the member gathers' registers
 // took waves from every plain plan (normed rows, D = 64: 105 registers -> 80,
 // 8 x 689 tokens of 16 heads 14.8 -> 12.3 us; fused rows 140 -> 69; plain
@@ -580,7 +582,7 @@ __device__ __forceinline__ void put_v(uint8_t* vt, int ch, int kl, const float* 
 // 41.2); without a fold that cost 2 us in 36 at 4096 tokens, and at D = 64 0.4
 // in 12. Four waves a SIMD is asked for where the registers land just above
 // that line.
-template <int D, bool LN, bool QKV, bool MERGE, bool EARLY>
+template <int D, bool LN, bool QKV, int MERGE, bool EARLY>
 __global__ __launch_bounds__(256, MERGE && (LN || D == 128) ? 1 : 4)
 void sage_quant_kv(const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, const float* __restrict__ ln,
                    float* __restrict__ stats, int8_t* __restrict__ k8, float* __restrict__ k_scale,
@@ -804,40 +806,42 @@ void sage_quant_kv(const uint16_t* __restrict__ k, const uint16_t* __restrict__ 
 #pragma unroll
             for (int e = 0; e < 8; e++) ks[e] = vs[e] = 0.f;
             // Member y nx + x is token base + y grid_w + x, and the members are
-            // summed in that order. A row of the cell at a time (merge is 2 or
-            // 4), its loads issued together, and only the rows the key has:
-            // one member at a time each wave waited out up to sixteen load
-            // latencies a key, dense keys' included (40 frames of 880 tokens,
-            // 16 heads, merge 4: 35.6 -> 27.1 us, 4.2 TB/s; two rows at a time
-            // 46.9, their registers leave two waves a SIMD). The norm's sums
-            // are over the D/8 lanes of one key, which run the same rows.
+            // summed in that order. A row of the cell at a time, its loads
+            // issued together, and only the rows the key has: one member at a
+            // time each wave waited out up to sixteen load latencies a key,
+            // dense keys' included. MERGE is the stride, so a row's loads take
+            // no more registers than it has members (stride 2 in rows of up to
+            // four left three waves a SIMD at head dim 128, not four). prepare,
+            // 40 frames of 689 tokens of 8 heads, us, members one at a time /
+            // rows of up to four / rows of the stride: D 64 stride 2 37.0 /
+            // 36.6 / 36.6, stride 4 57.7 / 47.2 / 41.0; D 128 stride 2 61.9 /
+            // 70.0 / 59.1, stride 4 95.4 / 75.0 / 65.1. The norm's sums are
+            // over the D/8 lanes of one key, which run the same rows.
             const uint16_t* kp = k + b * g.k_sb + (long long)base * g.k_st + hk * g.k_sh + ch * 8;
             const uint16_t* vp = v + b * g.v_sb + (long long)base * g.v_st + hk * g.v_sh + ch * 8;
             for (int y = 0; y * nx < cnt; y++) {
-                uint4 kr[4], vr[4];
+                uint4 kr[MERGE], vr[MERGE];
 #pragma unroll
-                for (int x = 0; x < 4; x++)
-                    if (x < g.merge) {
-                        const long long off = (long long)y * g.grid_w + x;
-                        const bool mok = x < nx && y * nx + x < cnt;
-                        kr[x] = load16(kp + off * g.k_st, mok);
-                        vr[x] = load16(vp + off * g.v_st, mok);
-                    }
+                for (int x = 0; x < MERGE; x++) {
+                    const long long off = (long long)y * g.grid_w + x;
+                    const bool mok = x < nx && y * nx + x < cnt;
+                    kr[x] = load16(kp + off * g.k_st, mok);
+                    vr[x] = load16(vp + off * g.v_st, mok);
+                }
 #pragma unroll
-                for (int x = 0; x < 4; x++)
-                    if (x < g.merge) {
-                        float fk[8], fv[8];
-                        unpack8(kr[x], fk, f16);
-                        unpack8(vr[x], fv, f16);
-                        if (LN) layernorm8<D>(fk, ln + 2 * D, ln + 3 * D, ch, g.ln_eps);
-                        if (x < nx && y * nx + x < cnt) {
+                for (int x = 0; x < MERGE; x++) {
+                    float fk[8], fv[8];
+                    unpack8(kr[x], fk, f16);
+                    unpack8(vr[x], fv, f16);
+                    if (LN) layernorm8<D>(fk, ln + 2 * D, ln + 3 * D, ch, g.ln_eps);
+                    if (x < nx && y * nx + x < cnt) {
 #pragma unroll
-                            for (int e = 0; e < 8; e++) {
-                                ks[e] += fk[e];
-                                vs[e] += fv[e];
-                            }
+                        for (int e = 0; e < 8; e++) {
+                            ks[e] += fk[e];
+                            vs[e] += fv[e];
                         }
                     }
+                }
             }
             const float rc = cnt > 0 ? 1.0f / (float)cnt : 0.f;
             float vq[8];
@@ -970,16 +974,20 @@ static hipError_t launch_prologue_d(const uint16_t* q, const uint16_t* k, const 
                            w.v8, w.kbias, fold ? w.part : nullptr, g, qa);
     };
     if (g.merge > 1) {
-        quant(std::true_type{}, std::false_type{});
+        if (QKV || g.merge == 4)
+            quant(std::integral_constant<int, 4>{}, std::false_type{});
+        else
+            quant(std::integral_constant<int, QKV ? 4 : 2>{}, std::false_type{});
         return hipGetLastError();
     }
+    using Plain = std::integral_constant<int, 0>;
     if constexpr (D == 128 && !QKV) {
         if (fold) {
-            quant(std::false_type{}, std::true_type{});
+            quant(Plain{}, std::true_type{});
             return hipGetLastError();
         }
     }
-    quant(std::false_type{}, std::false_type{});
+    quant(Plain{}, std::false_type{});
     return hipGetLastError();
 }
 
