@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256, D == 64 ? (MERGE ? 3 : 4) : (HET ? 3 : 2)) voi
     constexpr int BN = ATTN_BN, KS = D / 32, DT = D / 32, TILE = BN * D, KCPR = D / 16;
     constexpr int NL = TILE / 1024;  // 1 KB copies a tile
     constexpr bool ONE = HET && D == 128;
-    __shared__ __attribute__((aligned(16))) uint8_t ldsK[KEY_WAVES * TILE];
+    __shared__ __attribute__((aligned(128))) uint8_t ldsK[KEY_WAVES * TILE];
     __shared__ __attribute__((aligned(16))) uint8_t ldsV2[ONE ? 16 : KEY_WAVES * TILE];
     uint8_t* const ldsV = ONE ? ldsK : ldsV2;
     // The first sweep's maxima before shares 1 .. S - 1, [share - 1][wave][lane].
@@ -274,11 +274,30 @@ __global__ __launch_bounds__(256, D == 64 ? (MERGE ? 3 : 4) : (HET ? 3 : 2)) voi
 
     auto qk = [&](const uint8_t* kp, v16i (&s)[2]) __attribute__((always_inline)) {
         uint4 ka[2][KS];
+        // ONE: the operands of one row lie at koff[0] ^ 32 ks (2 ks + half is 2 ks
+        // ^ half, and tiles are 128-byte aligned), so one address is kept and the
+        // others are formed where they are read: kept as well, two registers
+        // went to scratch memory (272 to 816 tiles of 996 to 17764 keys: 0
+        // to 6.5% slower).
+        [[maybe_unused]] uint32_t k0 = 0;
+        if constexpr (ONE) {
+            k0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)kp + (uint32_t)koff[0];
+            opaque_vgpr(k0);
+        }
 #pragma unroll
         for (int t = 0; t < 2; t++) {
 #pragma unroll
-            for (int ks = 0; ks < KS; ks++)
-                ka[t][ks] = *reinterpret_cast<const uint4*>(kp + 16 * 32 * t * KCPR + koff[ks]);
+            for (int ks = 0; ks < KS; ks++) {
+                if constexpr (ONE) {
+#if defined(__HIP_DEVICE_COMPILE__)  // (an LDS pointer has 32 bits there)
+                    typedef unsigned u4 __attribute__((ext_vector_type(4)));
+                    const u4 w = *(__attribute__((address_space(3))) const u4*)((k0 ^ (uint32_t)(32 * ks)) + 16 * 32 * t * KCPR);
+                    ka[t][ks] = make_uint4(w.x, w.y, w.z, w.w);
+#endif
+                } else {
+                    ka[t][ks] = *reinterpret_cast<const uint4*>(kp + 16 * 32 * t * KCPR + koff[ks]);
+                }
+            }
             // (Three waves a SIMD at head dim 128: one sub-tile's operands at a time.)
             if (!ONE && t == 0) continue;
 #pragma unroll

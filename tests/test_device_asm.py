@@ -9,10 +9,14 @@ whenever the register allocator parks SGPRs in lanes of a vector register, so
 the source alone does not show it: the test compiles the unit as the build
 does and reads the assembly.
 
+Every attention kernel that a call can launch keeps the waves a SIMD it is
+laid out for and uses no scratch memory, by the compiler's own account of it.
+
 A forward call may write its output over Q, so the attention kernels that read
 the 16-bit queries promise no aliasing for neither of the two pointers."""
 from __future__ import annotations
 
+import functools
 import re
 import subprocess
 
@@ -64,13 +68,12 @@ def sgpr_hazards(asm: str, need: int = WAIT_STATES) -> list:
     return found
 
 
-def assembly(unit: str, tmp_path, *flags: str) -> str:
+@functools.lru_cache(maxsize=None)
+def assembly(unit: str, *flags: str) -> str:
     src, obj, extra = next(u for u in hip_build.UNITS if u[1] == unit)
-    out = tmp_path / (obj + ".s")
     cmd = [hip_build.HIPCC, *hip_build.COMMON, *extra, "-x", "hip", "--cuda-device-only", "-S", *flags,
-           str(hip_build.CSRC / src), "-o", str(out)]
-    subprocess.run(cmd, check=True, capture_output=True, timeout=300)
-    return out.read_text()
+           str(hip_build.CSRC / src), "-o", "-"]
+    return subprocess.run(cmd, check=True, capture_output=True, text=True, timeout=300).stdout
 
 
 def test_the_scan_sees_a_short_wait():
@@ -92,19 +95,19 @@ def test_only_these_units_load_in_inline_assembly():
 
 
 @pytest.mark.parametrize("unit", UNITS_WITH_ASM)
-def test_vector_memory_waits_for_its_base(unit, tmp_path):
-    asm = assembly(unit, tmp_path)
+def test_vector_memory_waits_for_its_base(unit):
+    asm = assembly(unit)
     assert "global_load_lds_dwordx4" in asm
     found = sgpr_hazards(asm)
     assert not found, f"{unit}: SGPR read too soon after a vector write: {found[:8]}"
 
 
 @pytest.mark.parametrize("unit", UNITS_WITH_ASM)
-def test_m0_belongs_to_the_asm_statements(unit, tmp_path):
+def test_m0_belongs_to_the_asm_statements(unit):
     """The copies write M0 (their LDS base) without the compiler's knowledge:
     nothing it generates in the unit may hold a value there."""
     inside, other = False, []
-    for n, line in enumerate(assembly(unit, tmp_path).splitlines(), 1):
+    for n, line in enumerate(assembly(unit).splitlines(), 1):
         if "ASMSTART" in line or "ASMEND" in line:
             inside = "ASMSTART" in line
         elif not inside and re.search(r"\bm0\b", line.split(";")[0]):
@@ -113,10 +116,10 @@ def test_m0_belongs_to_the_asm_statements(unit, tmp_path):
 
 
 @pytest.mark.parametrize("unit", ["sage_attention.hip.o", "sage_attention_merged.hip.o"])
-def test_queries_and_output_may_alias(unit, tmp_path):
+def test_queries_and_output_may_alias(unit):
     """sage_attn<D, CAUSAL, MERGE, QF = true>(q, ..., out, geometry): the host
     launches it with out = q (q_readable_beside)."""
-    ir = assembly(unit, tmp_path, "-emit-llvm", "-Xclang", "-disable-llvm-passes")
+    ir = assembly(unit, "-emit-llvm", "-Xclang", "-disable-llvm-passes")
     seen = 0
     for args in re.findall(r"define [^@\n]*@_ZN4sage9sage_attnILi\d+ELb[01]ELb[01]ELb1EE\w*\(([^\n]*?)\) #", ir):
         ptrs = [a for a in args.split(", ") if "ptr" in a and "byref" not in a]
@@ -126,3 +129,38 @@ def test_queries_and_output_may_alias(unit, tmp_path):
         assert all("noalias" in p for p in ptrs[3:8])  # codes, scales and statistics: read only
         seen += 1
     assert seen == (2 if "merged" in unit else 4)
+
+
+# VGPRs of the waves a SIMD each family is laid out for (512 a lane, in blocks
+# of 8): 128 for four, 168 for three, 256 for two. Template arguments after the
+# head dim: CAUSAL, MERGE, QF; CAUSAL, MERGE, shares, whole tiles beside them;
+# CAUSAL.
+WAVES = {
+    r"9sage_attnILi64E": 128,
+    r"9sage_attnILi128ELb[01]ELb0E": 168,
+    r"9sage_attnILi128ELb0ELb1E": 256,
+    r"14sage_attn_keysILi64ELb[01]ELb0E": 128,
+    r"14sage_attn_keysILi64ELb0ELb1E": 168,
+    r"14sage_attn_keysILi128ELb[01]ELb[01]ELi[24]ELb0E": 256,
+    r"14sage_attn_keysILi128ELb0ELb0ELi4ELb1E": 168,
+    r"15sage_attn_splitILi(64|128)E": 128,
+}
+KERNELS = {"sage_attention.hip.o": 12, "sage_attention_merged.hip.o": 4, "sage_attn_keys.hip.o": 10}
+
+
+@pytest.mark.parametrize("unit", sorted(KERNELS))
+def test_attention_kernels_fit(unit):
+    meta = assembly(unit).split(".amdgpu_metadata")[1]
+    kernels = re.split(r"\n  - ", meta)
+    seen = 0
+    for k in kernels:
+        name = re.search(r"\.name:\s+(\S*sage_attn\S*)", k)
+        if not name:
+            continue
+        get = lambda f: int(re.search(rf"\.{f}:\s+(\d+)", k).group(1))  # noqa: E731
+        limit = [v for pat, v in WAVES.items() if re.search(pat, name.group(1))]
+        assert len(limit) == 1, name.group(1)
+        assert get("private_segment_fixed_size") == 0 and get("vgpr_spill_count") == 0, name.group(1)
+        assert get("vgpr_count") <= limit[0], (name.group(1), get("vgpr_count"))
+        seen += 1
+    assert seen == KERNELS[unit]
