@@ -951,7 +951,7 @@ static hipError_t resources_of(int head_dim, int* regs, int* spill, int* lds) {
 //               144, N 1000: 37.1 / 38.3             160, N 2020: 53.9 / 52.8  160, N 4068: 82.1 / 77.9
 // A causal tile's keys end at its queries, so causal grids carry half the work
 // and longer tails (whole / two shares / four):
-//   D 64        160, N 356: 21.3 / 20.3 / 19.8       222: 21.6 / 20.7 / 21.6   320, N 740: 31.3 / 28.4 / 30.9
+//   D 64        192, N 740: 25.2 / 22.9 / 21.4       208, N 228: 19.6 / 19.3 / 19.6   312, N 740: 29.8 / 28.2 / 30.7
 //               400, N 740: 31.4 / 32.7 / 33.5       400, N 1000: 37.5 / 38.9 / 35.0
 //               440, N 2532: 58.1 / 56.6 / 53.7      480, N 2532: 50.9 / 50.8 / 51.0
 //               480, N 3044: 62.1 / 65.6 / 63.6      480, N 4068: 87.9 / 77.8 / 76.0
@@ -981,18 +981,18 @@ static hipError_t resources_of(int head_dim, int* regs, int* spill, int* lds) {
 //         32 over 768, N 228: 38.2 / 38.3     64, N 484: 45.7 / 45.2    112, N 996: 58.4 / 58.6   108, N 1508: 73.2 / 72.0
 //         64 over 1024, N 484: 54.6 / 54.3    80, N 1508: 87.6 / 86.8
 //         72 over 1280, N 1000: 81.7 / 83.2   64, N 1508: 102.4 / 100.8 64 over 1536, N 1000: 92.2 / 93.4, 2020: 139.6 / 137.2
-//   D 128 r 64 over 256, N 100: 32.8 / 31.4   88, N 1000: 50.6 / 51.0   80, N 10724: 231 / 217   104, N 3044: 92.7 / 93.8
-//         32 over 512, N 484: 56.3 / 56.7     64, N 1000: 69.6 / 68.5   72, N 1000: 69.5 / 73.4   64, N 3044: 124.7 / 117.1
-//         32 over 768, N 484: 74.5 / 75.1     64, N 1000: 91.3 / 90.5   80, N 1000: 91.8 / 97.2   48, N 3044: 167 / 153
-//         32 over 1024, N 2020: 153.9 / 156.2 32, N 3044: 200.5 / 197.2 56, N 3044: 200.6 / 201.3
-//         16 over 1280, N 3044: 234.0 / 228.5 64 over 1536, N 5092: 404 / 396 (runs of one side differ by 8%)
+//   D 128 r 64 over 256, N 100: 32.8 / 31.4   88, N 1000: 50.6 / 51.0   80, N 3044: 91.9 / 89.2   96, N 5604: 142 / 135
+//         32 over 512, N 484: 56.3 / 56.7     64, N 1000: 69.6 / 68.5   72, N 1000: 69.5 / 73.4   88, N 12772: 387 / 358
+//         32 over 768, N 484: 74.5 / 75.1     64, N 1000: 91.3 / 90.5   80, N 2020: 128.9 / 130.8 66, N 17764: 700 / 645
+//         32 over 1024, N 3044: 200 / 195     32, N 4068: 244 / 250     56, N 3044: 200 / 213     32, N 5604: 314 / 301
+//         32 over 1280, N 2020: 179.8 / 180.2 64, N 4068: 291 / 288     32 over 1536, N 2020: 207.5 / 208.5, 4068: 336 / 329
 // The tile of the context's Config does not matter here: it picks a layout,
 // never a result.
 KeySplit key_split(int head_dim, long long n, int heads, int kblocks, int merge, bool causal) {
     const bool wide = head_dim == 128;
     if (merge > 1) return {n <= (wide ? (merge == 2 ? 128 : 104) : (merge == 2 ? 224 : 176)) ? 2 : 0, 0};
     if (causal && !wide) {
-        if (kblocks < 16) return {n <= 176 ? 4 : n <= 320 ? 2 : 0, 0};
+        if (kblocks < 16) return {n <= 200 ? 4 : n <= 320 ? 2 : 0, 0};
         return {n <= (kblocks >= 56 && heads >= 5 ? 480 : 448) ? 4 : 0, 0};
     }
     if (causal) {
@@ -1009,7 +1009,7 @@ KeySplit key_split(int head_dim, long long n, int heads, int kblocks, int merge,
     };
     static constexpr Line LINES[2][6][2] = {
         {{{64, 1}, {176, 8}}, {{64, 1}, {136, 8}}, {{80, 8}, {112, 24}}, {{64, 8}, {80, 24}}, {{0, 0}, {80, 24}}, {{0, 0}, {64, 32}}},
-        {{{64, 1}, {96, 48}}, {{64, 16}, {64, 16}}, {{64, 16}, {64, 16}}, {{0, 0}, {32, 48}}, {{0, 0}, {32, 48}}, {{0, 0}, {0, 0}}}};
+        {{{64, 1}, {96, 48}}, {{64, 16}, {96, 64}}, {{64, 16}, {96, 48}}, {{0, 0}, {32, 80}}, {{0, 0}, {64, 64}}, {{0, 0}, {64, 64}}}};
     for (const Line& l : LINES[wide][f - 1])
         if (r <= l.most && kblocks >= l.blocks) return {4, (int)(n - r)};
     return {0, 0};

@@ -329,11 +329,14 @@ SPLITS = [
     ((128, 288, 72, 8, 1, True), (0, 0)),      # short keys: 40.9, 36.7
     ((64, 460, 2, 460, 1, True), (0, 0)),      # 457, 415
     ((64, 480, 15, 64, 1, True), (4, 0)),
+    ((64, 200, 100, 3, 1, True), (4, 0)),      # 15.0, 16.1 (two shares)
     ((64, 288, 48, 12, 1, True), (2, 0)),
     ((128, 144, 144, 2, 1, False), (0, 0)),    # 28.0, 24.3
     ((128, 160, 5, 64, 1, False), (4, 0)),
     ((128, 584, 73, 16, 1, False), (0, 0)),    # 73.3, 69.1: over three workgroups a CU
     ((128, 576, 72, 16, 1, False), (4, 512)),
+    ((128, 834, 6, 278, 1, False), (4, 768)),  # 645, 700
+    ((128, 848, 53, 32, 1, False), (0, 0)),    # 130.8, 128.9
     ((128, 580, 290, 4, 1, False), (0, 0)),    # 56.0, 49.9
     ((64, 1060, 530, 4, 1, False), (0, 0)),
     ((64, 352, 16, 44, 1, False), (4, 256)),
