@@ -5,13 +5,17 @@ layouts, QK LayerNorm, PvAccum::F16, smoothing off, custom softmax scales,
 strided Q/K/V layouts). Each case: the prologue bit-exact against the oracle
 and the attention within the north-star gate of the reference arithmetic
 (cos >= 0.999; max-abs 2e-2 plus half an output rounding step) and no
-further from f64 than that arithmetic."""
+further from f64 than that arithmetic. The problems as drawn have few query
+tiles and run the keys-split kernels; each runs again with its heads
+multiplied until the whole-key kernels take it."""
 from __future__ import annotations
+
+import dataclasses
 
 import numpy as np
 import pytest
 
-from sage_gpu_helpers import assert_prologue_equal, gather_rows, run, sample_rows
+from sage_gpu_helpers import assert_prologue_equal, gather_rows, run, sample_rows, split_of
 from test_gpu_parity import COS_MIN, COS_SLACK, MAX_ABS as ABS_MAX, REL_L2_SLACK
 
 pytestmark = pytest.mark.gpu
@@ -57,6 +61,16 @@ def _case(oracle, i: int):
     return p, gen, q_layout, out_dtype
 
 
+def _whole(p):
+    """The problem with the smallest multiple of its heads (KV heads alike)
+    that the whole-key kernels take."""
+    for m in range(1, 600):
+        w = dataclasses.replace(p, heads=p.heads * m, kv_heads=p.kv_heads * m)
+        if split_of(w)[0] == 0:
+            return w
+    raise AssertionError(p)
+
+
 def _check(oracle, p, want, o, rows, q, k, v, out_dtype, label):
     """The north-star gate against the emulated reference arithmetic, per
     element against its fp32 output: |ours - emu| <= 2e-2 plus half a step of
@@ -78,9 +92,12 @@ def _check(oracle, p, want, o, rows, q, k, v, out_dtype, label):
     assert e64["rel_l2"] <= emu64["rel_l2"] * 1.02 + REL_L2_SLACK, (e64, emu64)
 
 
-@pytest.mark.parametrize("i", range(CASES))
-def test_random_problem(oracle, torch_gpu, i):
+@pytest.mark.parametrize("i,whole", [(i, False) for i in range(CASES)] + [(i, True) for i in range(CASES)])
+def test_random_problem(oracle, torch_gpu, i, whole):
     p, gen, q_layout, out_dtype = _case(oracle, i)
+    assert split_of(p)[0] > 0
+    if whole:
+        p = _whole(p)
     print(f"case {i}: B{p.batch} H{p.heads}/{p.hk} N{p.tokens} D{p.head_dim} dtype {p.dtype} out {out_dtype} "
           f"causal {p.causal} merge {p.merge} {p.layout if p.merge > 1 else ''} ln {p.ln is not None} "
           f"pv16 {p.pv16} smooth {p.smooth_k} scale {p.softmax_scale} layout {q_layout}", flush=True)
@@ -88,4 +105,5 @@ def test_random_problem(oracle, torch_gpu, i):
     pro, o = run(torch_gpu, p, q, k, v, out_dtype=out_dtype, q_layout=q_layout)
     want = oracle.prologue(p, q, k, v)
     assert_prologue_equal(pro, want)
-    _check(oracle, p, want, o, sample_rows(p.tokens, 256, seed=i), q, k, v, out_dtype, f"case {i}")
+    count = max(8, 4096 // (p.batch * p.heads)) if whole else 256
+    _check(oracle, p, want, o, sample_rows(p.tokens, count, seed=i), q, k, v, out_dtype, f"case {i}")

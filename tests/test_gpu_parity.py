@@ -14,7 +14,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from sage_gpu_helpers import assert_prologue_equal, gather_rows, run, sample_rows, tile_rows
+from sage_gpu_helpers import assert_prologue_equal, gather_rows, run, sample_rows, split_of, tile_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -92,8 +92,11 @@ def test_small_cases(oracle, torch_gpu, name):
     _check_attention(oracle, p, want, o, rows, q, k, v, name)
 
 
+# Heads of 333 causal tokens (three tiles each): few run the keys-split kernels,
+# 120 the whole-key ones.
+@pytest.mark.parametrize("heads", [3, 120])
 @pytest.mark.parametrize("d", [64, 128])
-def test_zero_scales(oracle, torch_gpu, d):
+def test_zero_scales(oracle, torch_gpu, d, heads):
     """Degenerate scales: a K head constant over tokens (K smoothing leaves
     zeros, so every k_scale of that head is 0) and an all-zero 16-row Q group
     (q_scale 0), causal over a ragged tail. The attention kernel floors the
@@ -101,7 +104,8 @@ def test_zero_scales(oracle, torch_gpu, d):
     arithmetic has no floor, and a zero scale makes every logit of the row 0,
     so both give uniform attention over the visible keys. Codes bit-exact;
     outputs finite and at the gate on every row."""
-    p, g = oracle.Problem(1, 3, 333, d, causal=True), oracle.GenSpec(k_off_std=2.0, seed=41)
+    p, g = oracle.Problem(1, heads, 333, d, causal=True), oracle.GenSpec(k_off_std=2.0, seed=41)
+    assert (split_of(p)[0] == 0) == (heads == 120)
     q, k, v = oracle.generate(p, g)
     k[:, :, 0, :] = k[:, :1, 0, :]
     q[:, 32:48, 1, :] = 0
@@ -113,18 +117,20 @@ def test_zero_scales(oracle, torch_gpu, d):
     _check_attention(oracle, p, want, o, np.arange(p.tokens, dtype=np.int32), q, k, v, f"zero scales d{d}")
 
 
+@pytest.mark.parametrize("heads", [2, 120])
 @pytest.mark.parametrize("d", [64, 128])
-def test_tiny_q_scale_against_huge_k_scale(oracle, torch_gpu, d):
+def test_tiny_q_scale_against_huge_k_scale(oracle, torch_gpu, d, heads):
     """q_scale near 1e-23 against k_scale near 1e11 (bf16 Q ~ 1e-20, K ~ 1e13):
     their product, about 1e-12, is the reference's logit scale and must be used
     as is, with no floor on either factor (a floor of 1e-18 on q_scale would
     scale every logit up by about 1e5 and sharpen the rows far past the gate).
     Causal over a ragged tail, so masked -inf scores meet the product too."""
-    p = oracle.Problem(1, 2, 333, d, causal=True)
+    p = oracle.Problem(1, heads, 333, d, causal=True)
+    assert (split_of(p)[0] == 0) == (heads == 120)
     rng = np.random.default_rng(42)
-    qf = (rng.standard_normal((1, p.tokens, 2, d)) * 1e-20).astype(np.float32)
-    kf = (rng.standard_normal((1, p.tokens, 2, d)) * 1e13).astype(np.float32)
-    vf = rng.standard_normal((1, p.tokens, 2, d)).astype(np.float32)
+    qf = (rng.standard_normal((1, p.tokens, heads, d)) * 1e-20).astype(np.float32)
+    kf = (rng.standard_normal((1, p.tokens, heads, d)) * 1e13).astype(np.float32)
+    vf = rng.standard_normal((1, p.tokens, heads, d)).astype(np.float32)
     q, k, v = (oracle.encode16(x, p.dtype) for x in (qf, kf, vf))
     pro, o = run(torch_gpu, p, q, k, v)
     want = oracle.prologue(p, q, k, v)
@@ -221,14 +227,17 @@ def test_v_negative_zeros(oracle, torch_gpu, smooth_v, d):
         assert np.all(codes[:, :, t % 7 == 3, 16:] == 0x00)
 
 
+@pytest.mark.parametrize("heads", [4, 120])
 @pytest.mark.parametrize("d", [64, 128])
-def test_reference_tiles_give_identical_outputs(oracle, torch_gpu, d):
+def test_reference_tiles_give_identical_outputs(oracle, torch_gpu, d, heads):
     """Every tile the reference accepts (Tile::validate, mod.rs:158-167) runs; the
     reference's own defaults (Tile::DEFAULT {4,2,3}, Tile::D128 {4,1,3}) and other
-    accepted tiles give bit-identical codes and outputs (the tile only tunes)."""
+    accepted tiles give bit-identical codes and outputs (the tile only tunes),
+    where it picks a layout (120 heads) and where it picks none (4)."""
     import spl_sage as S
 
-    p, g = oracle.Problem(1, 4, 333, d, kv_heads=2, causal=True), oracle.GenSpec(k_off_std=2.0, seed=31)
+    p, g = oracle.Problem(1, heads, 333, d, kv_heads=2, causal=True), oracle.GenSpec(k_off_std=2.0, seed=31)
+    assert (split_of(p)[0] == 0) == (heads == 120)
     q, k, v = oracle.generate(p, g)
     pro0, o0 = run(torch_gpu, p, q, k, v)
     assert S.Config.for_head_dim(d).tile == (S.Tile.D128 if d == 128 else S.Tile.DEFAULT)

@@ -47,8 +47,10 @@ KERNEL_VGPR_LIMITS = {(64, "dense"): 128, (64, "causal"): 128, (64, "merged"): 1
 
 @pytest.mark.parametrize("d,kernel", sorted(KERNEL_VGPR_LIMITS))
 def test_gpu_every_attention_kernel_fits(torch_gpu, d, kernel):
-    """Every attention kernel (dense, causal, merged; both head dims) is free of
-    spills and keeps the waves a SIMD it is built for."""
+    """The attention kernels that the library reports (dense, causal, merged; both
+    head dims) are free of spills and keep the waves a SIMD they are built for.
+    (test_device_asm.py holds every kernel a call can launch: these, their
+    variants that quantise their own queries, and the keys-split ones.)"""
     import spl_sage as S
 
     regs, spill, lds = S.SageAttention(None, d).attn_kernel_resources(kernel)
