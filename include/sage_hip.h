@@ -67,9 +67,13 @@ typedef enum sage_pv_accum { SAGE_PV_F32 = 0, SAGE_PV_F16 = 1 } sage_pv_accum;
  * behind) over the same 128 queries; every other tile, the defaults included,
  * runs four wave64s of 32 queries, each doing the whole block. Both
  * double-buffer K and V. KV-merged attention always runs the four-wave
- * layout. Grids of too few query tiles to fill the chip run, under every tile,
- * a third layout that splits the keys over a workgroup's waves; its outputs
- * differ from the others' by the order of fp32 sums alone. */
+ * layout. Grids of too few query tiles to fill the chip, or of a few over a
+ * whole number a CU, run, under every tile, a third layout that splits the keys
+ * of some or all tiles over a workgroup's waves; its outputs differ from the
+ * others' by the order of fp32 sums alone. Which tiles it takes depends on the
+ * batch, the heads, the tokens and the plan's kind, never on the data: the same
+ * call gives the same bits, but a head's last bits can differ between a call of
+ * one batch item and a call of several. */
 typedef struct sage_tile {
     uint32_t warps;
     uint32_t m_tiles;
@@ -226,14 +230,15 @@ void* sage_stream(const sage_attention* s);                  /* mod.rs:636-638 *
 
 /* attn_resources (mod.rs:640-646): VGPRs per lane and scratch (spill) bytes
  * of the attention kernel, plus its static LDS bytes. The kernel is the one
- * the context's tile selects on grids that fill the chip: the eight-wave
- * layout for warps 8, else the four-wave kernel. */
+ * the context's tile selects for attend on grids that fill the chip: the
+ * eight-wave layout for warps 8, else the four-wave kernel. */
 sage_status sage_attn_resources(const sage_attention* s, int32_t* regs, int32_t* spill, int32_t* lds);
 
-/* The same for each attention kernel the context can launch (extension: the
- * reference reports its dense kernel only): SAGE_KERNEL_DENSE, _CAUSAL (the
- * causal extension) or _MERGED (KV merging, sg_attn_merge; always the
- * four-wave kernel). */
+/* The same for the kernels that attend launches on grids that fill the chip
+ * (extension: the reference reports its dense kernel only): SAGE_KERNEL_DENSE,
+ * _CAUSAL (the causal extension) or _MERGED (KV merging, sg_attn_merge; always
+ * the four-wave kernel). A forward call's variants, which quantise their own
+ * queries, and the keys-split kernels are not reported. */
 typedef enum sage_attn_kernel {
     SAGE_KERNEL_DENSE = 0,
     SAGE_KERNEL_CAUSAL = 1,

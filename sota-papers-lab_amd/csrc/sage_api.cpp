@@ -201,9 +201,9 @@ uint64_t sage_strides_extent(const sage_strides* s, uint64_t batch, uint64_t tok
 // Tile::validate (mod.rs:158-167): warps in {2, 4, 8}, m_tiles in {1, 2, 4},
 // stages 2..6, and the reference's rows per CTA (16 * m_tiles * warps)
 // dividing the 128-query tile. The tile picks the workgroup layout only
-// (attend_view): warps = 8 runs the eight-wave layout (score and output
-// waves) for dense and causal attention, every other tile the four-wave one;
-// outputs do not depend on it.
+// (attend_view): on grids that fill the chip warps = 8 runs the eight-wave
+// layout (score and output waves) for dense and causal attention, every other
+// tile the four-wave one; outputs do not depend on it.
 sage_status sage_tile_validate(const sage_tile* t) {
     if (!t) return fail(SAGE_ERR_INVALID, "null tile");
     const bool warps_ok = t->warps == 2 || t->warps == 4 || t->warps == 8;

@@ -106,9 +106,9 @@ __device__ __forceinline__ uint32_t lds_address(const void* p) {
 // forward, one frame 19.3 -> 18.8; sage_attn, whose blocks take longer, lost 2
 // to 3% to it at 384 and 768 tiles. It is older than every copy that the
 // caller counts, so those waits hold; the caller waits for it before it uses
-// the sink's memory. Only for heads of up to WARM_BYTES of K: an XCD's 4 MB L2 holds the K and V of
-// the heads its workgroups are on, and a longer head's would be gone again
-// before the sweep reaches them.
+// the sink's memory. Only for heads of up to WARM_BYTES of K: an XCD's 4 MB L2
+// holds the K and V of the heads its workgroups are on, and a longer head's
+// would be gone again before the sweep reaches them.
 constexpr long long WARM_BYTES = 3LL << 19;
 template <int D>
 __device__ __forceinline__ void warm_l2(const uint8_t* kg, const uint8_t* vg, long long bytes, int gi, uint32_t sink) {

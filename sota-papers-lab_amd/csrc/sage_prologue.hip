@@ -391,17 +391,6 @@ __global__ __launch_bounds__(256) void sage_prep(const uint16_t* __restrict__ q,
     }
 }
 
-// sage_quant.cu:163-206 (sg_finalize): even and odd tiles folded separately,
-// each in tile order, then combined. A workgroup takes FIN_CH channels of one
-// KV head, i.e. their 4 * FIN_CH (statistic, channel) columns. Its 256
-// threads stage up to FIN_CHUNK tiles of those columns in LDS with every load
-// of the chunk in flight at once; wave w then folds statistic w, one lane per
-// (channel, parity), in tile order, so the fold's operation is uniform across
-// the wave. A long sequence (VGGT's 1077 tiles a head) costs a few load
-// round trips instead of one per sixteen tiles. The workgroups of one head
-// share every 128-byte line of its partials, so they are dealt to one XCD
-// (the dispatcher deals linear ids round-robin over the 8 XCDs): each line
-// then comes from HBM into one L2 once.
 // A channel's K sum, V sum, V min and V max to its K mean, V mean, V scale and
 // 1 / V scale.
 __device__ __forceinline__ void finish_stats(float* st, const Geom& g) {
@@ -415,7 +404,7 @@ __device__ __forceinline__ void finish_stats(float* st, const Geom& g) {
     st[3] = 1.0f / st[2];
 }
 
-// The same fold inside every sage_quant_kv workgroup, for sequences of few
+// sage_finalize's fold inside every sage_quant_kv workgroup, for sequences of few
 // tiles: it saves a launch (about 2.5 us of the host's time and 2 to 4 of the
 // GPU's), and costs each workgroup its head's partials, q_tiles / 16 of the K
 // and V bytes it reads anyway, from L2. Whole prologue, us, three launches /
@@ -423,7 +412,11 @@ __device__ __forceinline__ void finish_stats(float* st, const Geom& g) {
 // 24.9 / 22.3, H 16 N 2048 (16 tiles) 13.4 / 11.9, B 8 H 16 N 2048 44.7 / 44.8,
 // N 2756 (22) 56.1 / 59.3; D 128 H 32 N 1000 18.1 / 16.7, B 8 H 16 N 1378 (11)
 // 59.5 / 58.0, H 16 N 2048 (16) 17.6 / 18.3, B 8 N 2756 103.9 / 109.3. So up to
-// 16 tiles at head dim 64 and 12 at 128 (two columns a thread).
+// 16 tiles at head dim 64 and 12 at 128 (two columns a thread). Normed rows: D 64
+// B 8 H 16 N 2038 52.2 / 51.9, N 2806 64.7 / 68.4; D 128 N 1398 74.0 / 74.4, N 2038
+// 94.6 / 97.5. The fused projection: D 64 N 2038 62.4 / 61.2, N 2806 81.3 / 82.0;
+// D 128 N 1398 83.1 / 78.8, N 2038 112 / 109, N 2806 148 / 152. Merged, H 16, one
+// frame of 689 tokens, stride 2: D 64 14.5 / 12.8, D 128 21.5 / 20.9.
 //
 // One thread a (statistic, channel) column, its loads independent, in
 // sage_finalize's order (even and odd tiles apart). `out` receives the four
@@ -467,6 +460,17 @@ __device__ __forceinline__ void fold_tiles(const float* __restrict__ part, float
     __syncthreads();
 }
 
+// sage_quant.cu:163-206 (sg_finalize): even and odd tiles folded separately,
+// each in tile order, then combined. A workgroup takes FIN_CH channels of one
+// KV head, i.e. their 4 * FIN_CH (statistic, channel) columns. Its 256
+// threads stage up to FIN_CHUNK tiles of those columns in LDS with every load
+// of the chunk in flight at once; wave w then folds statistic w, one lane per
+// (channel, parity), in tile order, so the fold's operation is uniform across
+// the wave. A long sequence (VGGT's 1077 tiles a head) costs a few load
+// round trips instead of one per sixteen tiles. The workgroups of one head
+// share every 128-byte line of its partials, so they are dealt to one XCD
+// (the dispatcher deals linear ids round-robin over the 8 XCDs): each line
+// then comes from HBM into one L2 once.
 constexpr int FIN_CH = 4;
 constexpr int FIN_CHUNK = 512;
 template <int D>
