@@ -29,10 +29,9 @@
 // is fetched over K(j) once QK^T has read it and lands during the softmax and
 // P.V; V(j + 1) over V(j) after P.V, landing during the next QK^T and softmax.
 // Four workgroups a CU at head dim 64 (registers; merged three), two at 128
-// (LDS). HET at
-// head dim 128 takes one buffer a wave for both tiles (ONE: V(j) over K(j), K(j
-// + 1) over V(j), their latency left to the other waves), three workgroups a
-// CU: its whole tiles fill the chip and want the waves.
+// (LDS). HET at head dim 128 takes one buffer a wave for both tiles (ONE: V(j)
+// over K(j), K(j + 1) over V(j), their latency left to the other waves), three
+// workgroups a CU: its whole tiles fill the chip and want the waves.
 #include "sage_attn_device.hpp"
 #include "sage_internal.hpp"
 

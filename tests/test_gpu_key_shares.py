@@ -10,6 +10,11 @@ running maximum that moves in the last share (token 0.9 N scaled up). The cases
 over the line keep the whole-key kernels' own masks and tails covered, the
 eight-wave layout among them. The gate is the fuzz test's: 2e-2 plus half an
 output step of the emulated reference arithmetic, and no further from f64.
+
+The softmax block is written out in sage_attn, in the eight-wave layout and in
+the keys-split kernels, and the probabilities must be the same E4M3 codes in all
+of them: the same heads are run in grids on either side of the line and compared
+far more tightly than any gate against the reference arithmetic.
 """
 from __future__ import annotations
 
@@ -80,3 +85,41 @@ def test_eight_waves_equal_four_over_the_line(oracle, torch_gpu, b, h, n, d, kw)
     _, base = run(torch_gpu, p, q, k, v, want_ws=False)
     _, o = run(torch_gpu, p, q, k, v, want_ws=False, tile=S.Tile(8, 1, 3))
     assert np.array_equal(o, base)
+
+
+# tokens, head dim, heads (split, whole), Problem arguments
+SAME = [
+    (1000, 64, 4, 58, {}),
+    (1000, 64, 34, 58, {}),                     # most tiles whole beside split ones
+    (1000, 128, 4, 21, dict(dtype=1)),
+    (1003, 128, 34, 43, {}),
+    (700, 64, 16, 72, dict(causal=True)),
+    (700, 64, 48, 72, dict(causal=True, dtype=1)),   # two shares
+    (1050, 128, 8, 40, dict(causal=True)),
+    (1050, 128, 30, 40, dict(causal=True)),     # two shares
+    (12 * 95, 64, 4, 26, dict(merge=2, layout=(12, 5, 9, 10, 1))),
+    (12 * 95, 128, 4, 15, dict(merge=4, layout=(12, 5, 9, 10, 0))),
+]
+
+
+@pytest.mark.parametrize("n,d,few,many,kw", SAME, ids=[f"n{c[0]}d{c[1]}h{c[2]}_{c[3]}" for c in SAME])
+def test_the_same_heads_split_and_whole(oracle, torch_gpu, n, d, few, many, kw):
+    """The two sides differ by the order of fp32 sums of up to N terms alone: l and
+    O move by some tens of roundings (64 * 2^-24 of the largest output, taken as
+    4e-6), so an output moves by that and, where it lies that close to a rounding
+    edge of the 16-bit type (4e-6 against steps of 2^-8 or 2^-9: 2e-3 of all),
+    one step more. Probabilities of another E4M3 grid (a share's own maximum
+    instead of the running one) move outputs by 2e-2 in the 2-norm and most of
+    them by a step; what is let through here is sqrt(2e-3) * 2^-8 = 2e-4."""
+    p, q, k, v = _problem(oracle, 1, many, n, d, kw, 300 + n + d)
+    f = oracle.Problem(1, few, n, d, **kw)
+    assert split_of(p)[0] == 0 and split_of(f)[0] > 0
+    _, whole = run(torch_gpu, p, q, k, v, want_ws=False)
+    _, split = run(torch_gpu, f, *(np.ascontiguousarray(x[:, :, :few]) for x in (q, k, v)), want_ws=False)
+    a, b = (oracle.decode16(x, p.dtype).astype(np.float64) for x in (whole[:, :, :few], split))
+    step = 2.0 ** (-7 if p.dtype == 0 else -10)  # the widest step of the type at 1
+    moved = np.abs(a - b)
+    print(f"{(moved > 0).mean():.2e} of outputs moved, at most {moved.max() / np.abs(a).max():.2e} of the largest")
+    assert np.all(moved <= 4e-6 * np.abs(a).max() + step * np.abs(a))
+    assert (moved > 0).mean() <= 2e-3
+    assert np.linalg.norm(a - b) <= 2e-4 * np.linalg.norm(a)
