@@ -51,19 +51,18 @@ constexpr int KEY_ROWS = 32;  // queries a group
 // after a vector instruction wrote it, the compiler keeps no such distance to
 // an asm statement, and a base restored from a vector register's lanes
 // (v_readlane) arrives right before it. A scalar read of that SGPR is
-// interlocked, and a scalar write needs no wait before the load. M0, the copies'
-// LDS base, needs one wait state before the load (s_nop); it is a reserved
-// register that cannot be named as clobbered, so a kernel that uses these
-// helpers has no other use of it.
+// interlocked, and a scalar write needs no wait before the load. The move is
+// also the one wait state that M0, the copies' LDS base, needs before the load.
+// (M0 is a reserved register that cannot be named as clobbered: a kernel that
+// uses these helpers has no other use of it.)
 // 4 KB, four copies of 64 lanes x 16 bytes: copy i reads base + 1024 i + even
 // (odd copies: + odd) and fills dst + 1024 i + 16 lane.
 __device__ __forceinline__ void copy_4k(const uint8_t* base, uint32_t even, uint32_t odd, uint32_t dst) {
 #if defined(__HIP_DEVICE_COMPILE__)
     const uint8_t* b;
     asm volatile(
-        "s_mov_b64 %0, %4\n\t"
         "s_mov_b32 m0, %1\n\t"
-        "s_nop 0\n\t"
+        "s_mov_b64 %0, %4\n\t"
         "global_load_lds_dwordx4 %2, %0\n\t"
         "global_load_lds_dwordx4 %3, %0 offset:1024\n\t"
         "global_load_lds_dwordx4 %2, %0 offset:2048\n\t"
@@ -78,9 +77,8 @@ __device__ __forceinline__ void copy_1k(const uint8_t* base, uint32_t off, uint3
 #if defined(__HIP_DEVICE_COMPILE__)
     const uint8_t* b;
     asm volatile(
-        "s_mov_b64 %0, %3\n\t"
         "s_mov_b32 m0, %1\n\t"
-        "s_nop 0\n\t"
+        "s_mov_b64 %0, %3\n\t"
         "global_load_lds_dwordx4 %2, %0"
         : "=&s"(b)
         : "s"(__builtin_amdgcn_readfirstlane((int)dst)), "v"(off), "s"(base)
@@ -92,9 +90,8 @@ __device__ __forceinline__ void copy_256(const uint8_t* base, uint32_t off, uint
 #if defined(__HIP_DEVICE_COMPILE__)
     const uint8_t* b;
     asm volatile(
-        "s_mov_b64 %0, %3\n\t"
         "s_mov_b32 m0, %1\n\t"
-        "s_nop 0\n\t"
+        "s_mov_b64 %0, %3\n\t"
         "global_load_lds_dword %2, %0"
         : "=&s"(b)
         : "s"(__builtin_amdgcn_readfirstlane((int)dst)), "v"(off), "s"(base)
