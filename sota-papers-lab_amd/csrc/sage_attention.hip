@@ -954,6 +954,9 @@ static hipError_t resources_of(int head_dim, int* regs, int* spill, int* lds) {
 
 // How the keys are split (KeySplit), by the number n of 128-query tiles, their
 // remainder r over whole multiples of the chip's 256 CUs, and the 64-key blocks.
+// Split kernels have a workgroup per 32 or 64 queries that exist, so for them a
+// ragged tile counts by its quarters (m; 25 KV heads of 308 causal tokens, 50
+// heads, head dim 128: 150 tiles, 500 workgroups, 30.2 us whole, 27.9 split).
 //
 // Few tiles. A tile is one wave a SIMD, and a lone wave takes 1.6 times the
 // chip's best time a block, so up to about n = 256 the chip is short of waves;
@@ -962,6 +965,10 @@ static hipError_t resources_of(int head_dim, int* regs, int* spill, int* lds) {
 // the prologue. They pay while their workgroups are resident at once (four a
 // CU at head dim 64, two at 128: 256 and 128 tiles of four shares) and, where
 // the keys are long enough for the loop to outweigh the rest, a little beyond.
+// One rule for every entry, so that a forward gives prepare and attend's bits:
+// the figures are of forwards, whose whole-key kernels make Q's codes; prepare
+// and attend (the fused projection, normed rows) put each line a little higher,
+// and where the two differ it stands where neither loses more than 3%.
 // A forward on the GPU, us, whole keys / split (graph replays, one box):
 //   D 64        96 tiles N 684: 23.5 / 18.4          192, N 100: 17.8 / 18.3   192, N 1000: 27.6 / 25.0
 //               224, N 484: 22.9 / 23.3              224, N 2020: 39.4 / 38.6  256, N 1000: 28.5 / 28.1
@@ -972,8 +979,9 @@ static hipError_t resources_of(int head_dim, int* regs, int* spill, int* lds) {
 //   D 64        192, N 740: 25.2 / 22.9 / 21.4       208, N 228: 19.6 / 19.3 / 19.6   312, N 740: 29.8 / 28.2 / 30.7
 //               400, N 740: 31.4 / 32.7 / 33.5       400, N 1000: 37.5 / 38.9 / 35.0
 //               440, N 2532: 58.1 / 56.6 / 53.7      480, N 2532: 50.9 / 50.8 / 51.0
-//               480, N 3044: 62.1 / 65.6 / 63.6      480, N 4068: 87.9 / 77.8 / 76.0
+//               480, N 3044: 62.1 / 65.6 / 63.6      459, N 3416: 71.7 / 67.1         480, N 4068: 87.9 / 77.8 / 76.0
 //   D 128       126, N 356: 27.7 / 24.7 / 23.9       159: 29.3 / 28.9 / 30.4   204, N 740: 36.1 / 36.1 / 38.1
+//               129 to 144, two shares: N 228 +1 to 3%, N 356 -7 to -1%, N 740 -7 to -1%
 //               208, N 1636: 48.8 / 43.4 / 43.2      248, N 1000: 40.0 / 39.3 / 43.0
 //               288, N 484: 36.7 / 40.9 / 42.7       288, N 2020: 70.8 / 63.7 / 66.3
 //               352, N 2764: 70.8 / 66.1 / 72.8      352, N 1000: 51.6 / 53.6 / 54.6
@@ -995,7 +1003,7 @@ static hipError_t resources_of(int head_dim, int* regs, int* spill, int* lds) {
 // 512 whole ones); short keys, and more whole tiles a CU, leave it less to gain
 // (whole / r split):
 //   D 64  r 64 over 256, N 100: 22.0 / 21.7   144, N 100: 23.5 / 24.9   176, N 484: 30.5 / 30.1   128, N 3044: 68.9 / 59.2
-//         64 over 512, N 228: 30.8 / 30.2     128, N 484: 37.4 / 37.3   128, N 1000: 47.8 / 45.6
+//         64 over 512, N 228: 30.8 / 30.2     128, N 484: 37.4 / 37.3   128, N 1000: 47.8 / 45.6   (136 is a second round)
 //         32 over 768, N 228: 38.2 / 38.3     64, N 484: 45.7 / 45.2    112, N 996: 58.4 / 58.6   108, N 1508: 73.2 / 72.0
 //         64 over 1024, N 484: 54.6 / 54.3    80, N 1508: 87.6 / 86.8
 //         72 over 1280, N 1000: 81.7 / 83.2   64, N 1508: 102.4 / 100.8 64 over 1536, N 1000: 92.2 / 93.4, 2020: 139.6 / 137.2
@@ -1006,36 +1014,47 @@ static hipError_t resources_of(int head_dim, int* regs, int* spill, int* lds) {
 //         32 over 1280, N 2020: 179.8 / 180.2 64, N 4068: 291 / 288     32 over 1536, N 2020: 207.5 / 208.5, 4068: 336 / 329
 // The tile of the context's Config does not matter here: it picks a layout,
 // never a result.
-KeySplit key_split(int head_dim, long long n, int heads, int kblocks, int merge, bool causal) {
+KeySplit key_split(int head_dim, int tokens, int heads, int kblocks, int merge, bool causal) {
     const bool wide = head_dim == 128;
-    if (merge > 1) return {n <= (wide ? (merge == 2 ? 128 : 104) : (merge == 2 ? 224 : 176)) ? 2 : 0, 0};
+    const long long n = ((long long)tokens + 127) / 128 * heads;
+    // (Of a key block or three there is nothing to share.)
+    const long long m = kblocks >= 4 ? (((long long)tokens + 31) / 32 * heads + 3) / 4 : n;
+    if (merge > 1) return {m <= (wide ? (merge == 2 ? 128 : 104) : (merge == 2 ? 224 : 192)) ? 2 : 0, 0};
     if (causal && !wide) {
-        if (kblocks < 16) return {n <= 200 ? 4 : n <= 320 ? 2 : 0, 0};
-        return {n <= (kblocks >= 56 && heads >= 5 ? 480 : 448) ? 4 : 0, 0};
+        if (kblocks < 16) return {m <= 200 ? 4 : m <= 320 ? 2 : 0, 0};
+        return {m <= (kblocks >= 52 && heads >= 5 ? 480 : 448) ? 4 : 0, 0};
     }
     if (causal) {
-        if (kblocks < 16) return {n <= 128 ? 4 : 0, 0};
-        return {n <= 208 ? 4 : n <= (heads >= 5 ? 288 : 256) ? 2 : 0, 0};
+        if (kblocks < 16) return {m <= 128 ? 4 : m <= 144 && kblocks >= 5 ? 2 : 0, 0};
+        return {m <= 208 ? 4 : m <= (heads >= 5 ? 288 : 256) ? 2 : 0, 0};
     }
-    if (n <= (wide ? (kblocks >= 32 ? 160 : 128) : (kblocks >= 16 ? 224 : 192))) return {4, 0};
+    if (m <= (wide ? (kblocks >= 24 ? 160 : 128) : (kblocks >= 16 ? 224 : 192))) return {4, 0};
     const long long f = n / 256, r = n % 256;
     if (f == 0 || f > 6 || r == 0) return {0, 0};
-    // [whole tiles a CU - 1]: the largest remainder that is split from so many
-    // key blocks on, for shorter keys and longer ones.
+    // [whole tiles a CU - 1]: the largest remainders that are split from so many
+    // key blocks on.
     struct Line {
         int most, blocks;
     };
-    static constexpr Line LINES[2][6][2] = {
-        {{{64, 1}, {176, 8}}, {{64, 1}, {136, 8}}, {{80, 8}, {112, 24}}, {{64, 8}, {80, 24}}, {{0, 0}, {80, 24}}, {{0, 0}, {64, 32}}},
-        {{{64, 1}, {96, 48}}, {{64, 16}, {96, 64}}, {{64, 16}, {96, 48}}, {{0, 0}, {32, 80}}, {{0, 0}, {64, 64}}, {{0, 0}, {64, 64}}}};
+    static constexpr Line LINES[2][6][3] = {{{{64, 1}, {96, 4}, {176, 8}},
+                                             {{64, 1}, {128, 8}},
+                                             {{32, 6}, {80, 8}, {112, 16}},
+                                             {{64, 8}, {80, 16}},
+                                             {{80, 16}},
+                                             {{64, 24}}},
+                                            {{{64, 1}, {96, 32}},
+                                             {{64, 8}, {96, 48}},
+                                             {{64, 12}, {96, 48}},
+                                             {{48, 48}},
+                                             {{64, 32}},
+                                             {{64, 64}}}};
     for (const Line& l : LINES[wide][f - 1])
         if (r <= l.most && kblocks >= l.blocks) return {4, (int)(n - r)};
     return {0, 0};
 }
 
 static KeySplit key_split(int head_dim, const Geom& g) {
-    return key_split(head_dim, (long long)g.q_tiles * g.heads * g.batch, g.heads * g.batch, g.kblocks, g.merge,
-                     g.flags & F_CAUSAL);
+    return key_split(head_dim, g.tokens, g.heads * g.batch, g.kblocks, g.merge, g.flags & F_CAUSAL);
 }
 
 // The whole-key four-wave kernels have the variant; the sage options' QK

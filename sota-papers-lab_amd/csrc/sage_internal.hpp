@@ -67,11 +67,11 @@ hipError_t launch_attention(int head_dim, const AttendBufs& w, const Geom& g, hi
 hipError_t launch_attention_merged(int head_dim, const AttendBufs& w, const Geom& g, hipStream_t s);
 // How launch_attention splits the keys: the shares a query group's keys are
 // split into (0: none), and the 128-query tiles left whole beside them.
-// tiles: of all heads and batch items, heads: over the batch.
+// heads: over the batch.
 struct KeySplit {
     int shares, whole;
 };
-KeySplit key_split(int head_dim, long long tiles, int heads, int kblocks, int merge, bool causal);
+KeySplit key_split(int head_dim, int tokens, int heads, int kblocks, int merge, bool causal);
 hipError_t launch_attention_keys(int head_dim, const KeySplit& k, const AttendBufs& w, const Geom& g, hipStream_t s);
 
 // Whether a forward call on this geometry leaves Q's codes to the attention

@@ -17,11 +17,11 @@ def v8_logical(raw: np.ndarray, b: int, g: int, tk_pad: int, d: int) -> np.ndarr
     return np.ascontiguousarray(x.transpose(0, 1, 2, 4, 3)).reshape(b, g, tk_pad, d)
 
 
-def key_split(head_dim: int, tiles: int, heads: int, kblocks: int, merge: int = 1, causal: bool = False) -> tuple:
+def key_split(head_dim: int, tokens: int, heads: int, kblocks: int, merge: int = 1, causal: bool = False) -> tuple:
     """(shares, whole tiles) of the library's own rule: shares 0 is the
     whole-key kernels (four or eight waves, by the Config's tile), shares
     without whole tiles the keys-split kernel, both the one that leaves most
-    tiles whole. tiles: 128-query tiles of all `heads` (batch x heads)."""
+    tiles whole. heads: batch x heads."""
     import ctypes as C
 
     from spl_sage import _abi
@@ -29,9 +29,9 @@ def key_split(head_dim: int, tiles: int, heads: int, kblocks: int, merge: int = 
     class Split(C.Structure):
         _fields_ = [("shares", C.c_int), ("whole", C.c_int)]
 
-    f = _abi.lib()._ZN4sage9key_splitEixiiib
-    f.restype, f.argtypes = Split, [C.c_int, C.c_longlong, C.c_int, C.c_int, C.c_int, C.c_bool]
-    r = f(head_dim, tiles, heads, kblocks, merge, causal)
+    f = _abi.lib()._ZN4sage9key_splitEiiiiib
+    f.restype, f.argtypes = Split, [C.c_int] * 5 + [C.c_bool]
+    r = f(head_dim, tokens, heads, kblocks, merge, causal)
     return r.shares, r.whole
 
 
@@ -42,7 +42,7 @@ def split_of(p) -> tuple:
     merge = S.KvMerge.Dense if p.merge == 1 else S.KvMerge.Pool(p.merge, S.FrameLayout(*p.layout))
     plan = S.Plan.new(S.Shape(p.batch, p.heads, p.tokens, p.kv_heads), merge)
     heads = p.batch * p.heads
-    return key_split(p.head_dim, plan.q_tiles() * heads, heads, plan.kblocks(), p.merge, bool(p.causal))
+    return key_split(p.head_dim, p.tokens, heads, plan.kblocks(), p.merge, bool(p.causal))
 
 
 def run(torch, p, q, k, v, out_dtype=None, q_layout="bthd", out_layout="bthd", want_ws=True, tile=None):

@@ -169,7 +169,7 @@ def test_merged_padding_keys_have_no_influence(oracle, torch_gpu, H, D):
     ws = sa.workspace(S.Shape(1, H, T), S.KvMerge.Pool(4, layout))
     plan = ws.plan()
     assert plan.tk_pad > plan.tk
-    assert (key_split(D, plan.q_tiles() * H, H, plan.kblocks(), 4)[0] == 0) == (H == 16)
+    assert (key_split(D, T, H, plan.kblocks(), 4)[0] == 0) == (H == 16)
     outs = []
     for poison in (False, True):
         out = torch_gpu.empty((1, T, H, D), dtype=torch_gpu.bfloat16, device="cuda")

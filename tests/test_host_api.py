@@ -337,16 +337,18 @@ SPLITS = [
     ((128, 576, 72, 16, 1, False), (4, 512)),
     ((128, 834, 6, 278, 1, False), (4, 768)),  # 645, 700
     ((128, 848, 53, 32, 1, False), (0, 0)),    # 130.8, 128.9
-    ((128, 580, 290, 4, 1, False), (0, 0)),    # 56.0, 49.9
+    ((128, 576, 288, 4, 1, False), (0, 0)),    # 51.5, 48.9
     ((64, 1060, 530, 4, 1, False), (0, 0)),
     ((64, 352, 16, 44, 1, False), (4, 256)),
     ((64, 640, 80, 16, 1, False), (4, 512)),   # 47.8, 45.6
-    ((64, 880, 110, 16, 1, False), (0, 0)),    # 58.6, 58.4
+    ((64, 880, 220, 8, 1, False), (0, 0)),     # 46.9, 46.1
     ((64, 876, 73, 24, 1, False), (4, 768)),   # 72.0, 73.2
+    ((64, 648, 81, 16, 1, False), (0, 0)),     # 136 over 512: a second round of workgroups
     ((128, 344, 43, 16, 1, False), (0, 0)),    # 51.0, 50.6
     ((128, 336, 4, 168, 1, False), (4, 256)),  # 231, 217
     ((128, 120, 20, 4, 4, False), (0, 0)),     # merged, stride 4: 49.2, 45.3
     ((64, 222, 37, 2, 4, False), (0, 0)),      # 35.2, 32.4
+    ((128, 132, 22, 12, 1, True), (2, 0)),     # 31.6, 33.0
     ((64, 222, 37, 4, 2, False), (2, 0)),
 ]
 
@@ -355,7 +357,17 @@ SPLITS = [
 def test_key_split_lines(S, args, want):
     from sage_gpu_helpers import key_split
 
-    assert key_split(*args) == want
+    d, tiles, heads, *rest = args
+    assert key_split(d, tiles // heads * 128, heads, *rest) == want
+
+
+def test_ragged_tiles_count_by_their_quarters(S):
+    """Split kernels have no workgroup for 32-query groups past the sequence."""
+    from sage_gpu_helpers import key_split
+
+    assert key_split(128, 308, 50, 5, 1, True) == (4, 0)   # ten groups a head, 125 tiles of them
+    assert key_split(128, 384, 50, 6, 1, True) == (0, 0)   # twelve: 150
+    assert key_split(64, 17, 450, 1, 1, False) == (0, 0)   # one key block: nothing to share
 
 
 def test_key_split_gives_what_the_kernels_are_built_for(S):
@@ -364,12 +376,13 @@ def test_key_split_gives_what_the_kernels_are_built_for(S):
     from sage_gpu_helpers import key_split
 
     for d in (64, 128):
-        for tiles in [*range(1, 2100), 1 << 20, 1 << 34]:
-            for heads in (1, 4, 5, 64):
-                for kb in (1, 4, 8, 16, 24, 32, 48, 56, 300):
-                    s, w = key_split(d, tiles, heads, kb, 1, False)
-                    assert (s, w) == (0, 0) or (s == 4 and w % 256 == 0 and w < tiles and (w or tiles < 256)), (d, tiles)
-                    s, w = key_split(d, tiles, heads, kb, 1, True)
-                    assert s in (0, 2, 4) and w == 0
-            for m in (2, 4):
-                assert key_split(d, tiles, 4, 8, m, False) in ((0, 0), (2, 0))
+        for heads in [*range(1, 2100, 7), 1 << 20]:
+            for tokens in (1, 33, 128, 200, 1000, 2040, 17776, 1 << 24):
+                kb, tiles = -(-tokens // 64), -(-tokens // 128) * heads
+                s, w = key_split(d, tokens, heads, kb, 1, False)
+                assert (s, w) == (0, 0) or (s == 4 and w % 256 == 0 and w < tiles), (d, tokens, heads)
+                assert not w or tiles - w < 256
+                s, w = key_split(d, tokens, heads, kb, 1, True)
+                assert s in (0, 2, 4) and w == 0
+                for m in (2, 4):
+                    assert key_split(d, tokens, heads, kb, m, False) in ((0, 0), (2, 0))
