@@ -590,38 +590,33 @@ __global__ __launch_bounds__(256, D == 64 ? 4 : (MERGE ? 2 : 3)) void sage_attn(
         // Pairs of outputs go through gfx950's packed converters
         // (v_cvt_pk_bf16_f32, v_cvt_pk_f16_f32: round to nearest even), one
         // uniform branch on the output type.
-        // A channel tile's statistics are loaded together ahead of its stores: the
-        // output may be Q, so the compiler moves no load over a store, and one load
-        // a group, each waited for, took 1.9 us of a one-block tile's 7.7 at head
-        // dim 128 (5.8 so). The next tile's ahead of this one's stores gain
-        // nothing more (2 x 4096 tokens: 403.4 us a forward, 398.5 so).
+        // The output may be Q, so the compiler moves no load over a store: the
+        // statistics of two groups of four channels are loaded ahead of their two
+        // stores. One group at a time a one-block tile waited out sixteen loads at
+        // head dim 128 (7.8 us, 6.4 in twos, 6.0 in fours); in fours the loads and
+        // stores of a full chip's tiles crowd (2 x 4096 tokens, us a forward: 409 /
+        // 410 / 414, 700 heads of 200 88.2 / 89.2 / 90.5).
         auto emit = [&](auto pack) __attribute__((always_inline)) {
-            float4 vs[2][4], vm[2][4];
-            auto load = [&](int dt) __attribute__((always_inline)) {
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const int d0 = 32 * dt + 8 * j + 4 * half_e;
-                    vs[dt & 1][j] = *reinterpret_cast<const float4*>(vscale + d0);
-                    vm[dt & 1][j] = *reinterpret_cast<const float4*>(vmean + d0);
+            for (int dt = 0; dt < DT; dt++)
+#pragma unroll
+                for (int j0 = 0; j0 < 4; j0 += 2) {
+                    float4 vs[2], vm[2];
+#pragma unroll
+                    for (int i = 0; i < 2; i++) {
+                        const int d0 = 32 * dt + 8 * (j0 + i) + 4 * half_e;
+                        vs[i] = *reinterpret_cast<const float4*>(vscale + d0);
+                        vm[i] = *reinterpret_cast<const float4*>(vmean + d0);
+                    }
+#pragma unroll
+                    for (int i = 0; i < 2; i++) {
+                        const int r = 4 * (j0 + i);
+                        uint2 w;
+                        w.x = pack(fmaf(o[dt][r] * inv, vs[i].x, vm[i].x), fmaf(o[dt][r + 1] * inv, vs[i].y, vm[i].y));
+                        w.y = pack(fmaf(o[dt][r + 2] * inv, vs[i].z, vm[i].z), fmaf(o[dt][r + 3] * inv, vs[i].w, vm[i].w));
+                        *reinterpret_cast<uint2*>(orow + 32 * dt + 8 * (j0 + i) + 4 * half_e) = w;
+                    }
                 }
-            };
-#pragma unroll
-            for (int dt = 0; dt < DT; dt++) {
-                load(dt);
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const float4 sv = vs[dt & 1][j], mv = vm[dt & 1][j];
-                    float y[4];
-                    y[0] = fmaf(o[dt][4 * j] * inv, sv.x, mv.x);
-                    y[1] = fmaf(o[dt][4 * j + 1] * inv, sv.y, mv.y);
-                    y[2] = fmaf(o[dt][4 * j + 2] * inv, sv.z, mv.z);
-                    y[3] = fmaf(o[dt][4 * j + 3] * inv, sv.w, mv.w);
-                    uint2 w;
-                    w.x = pack(y[0], y[1]);
-                    w.y = pack(y[2], y[3]);
-                    *reinterpret_cast<uint2*>(orow + 32 * dt + 8 * j + 4 * half_e) = w;
-                }
-            }
         };
         if (g.flags & F_OUT_F16)
             emit([](float a, float b) { return pack_f16x2(a, b); });
